@@ -56,8 +56,19 @@
 
 namespace tmx {
 
+// Occupancy: at head_dim 65-128 LDS (64 or 80 KB per workgroup) and the 168-256
+// VGPRs allow 2 waves per SIMD.  At head_dim <= 64 a workgroup takes 32 or 40 KB
+// and 104-164 VGPRs, so 3 or 4 fit; the tile loop is a serial chain per wave
+// (QK -> max -> exps -> PV), and a third wave fills its gaps.  The upper bound
+// matters as much as the lower one: (2, 2) makes the compiler round the VGPR
+// allocation up until a third wave does not fit.  A lower bound of 4 (128 VGPRs)
+// spills in every mixed instantiation.  B8 x 2048, 32/8 heads, head_dim 64, kernel
+// at (2, 2) / (3, 4) / (4, 4): block_m 64 mixed 227 / 199 / 223 us, fp16 mode 218 /
+// 190 / 191, int8 mode 217 / 187 / 189, mixed with int8 V 262 / 225 / 216; B8 x 4096
+// 891 / 764 / 781.
 template <int NW, int DP, int MODE, bool INT8V, bool DUMP, bool BIAS, bool SPLIT, bool GEN, bool PIPE = false>
-__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(NW * 64)
+__attribute__((amdgpu_waves_per_eu(DP <= 64 ? 3 : 2, DP <= 64 ? 4 : 2)))
 attn32_kernel(const AttnKArgs a) {
   static_assert(!SPLIT || (NW % 2 == 0 && !INT8V), "split workgroups: even wave count, fp16 V");
   static_assert(!PIPE || (NW == 4 && DP == 128 && !INT8V && !DUMP && !BIAS && !GEN),
