@@ -91,6 +91,16 @@ typedef struct tilemix_quant_params {
 int tilemix_quant_per_block_int8(const tilemix_quant_params* p, void* stream);
 
 /*
+ * The same for `count` (1 to 3) tensors in one launch, e.g. the K and V of a call
+ * or all of Q, K and V.  uniform_seqlen > 0: sequence b is tokens
+ * [b * uniform_seqlen, (b + 1) * uniform_seqlen) of every tensor; cu_seqlens and
+ * max_seqlen are then not read (cu_seqlens may be NULL), and cu_seqlens_scale is
+ * written if it is not NULL.  uniform_seqlen = 0: each tensor's own cu_seqlens.
+ */
+int tilemix_quant_per_block_int8_many(const tilemix_quant_params* p, int32_t count, int32_t uniform_seqlen,
+                                      void* stream);
+
+/*
  * Fused FP16/INT8-routed flash-attention prefill forward.
  * Replaces attn_fwd (attention/triton/tilemix.py:503-951) launched by
  * launch_prequantized (:1132-1337).  One launch computes, for every sequence z,

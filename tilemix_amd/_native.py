@@ -106,6 +106,7 @@ class RotaryParams(ctypes.Structure):
 
 EXPORTED_SYMBOLS = (
     "tilemix_quant_per_block_int8",
+    "tilemix_quant_per_block_int8_many",
     "tilemix_attn_fwd",
     "tilemix_attn_fwd_debug",
     "tilemix_rms_norm_f16",
@@ -141,6 +142,8 @@ def load_library(path: os.PathLike | str | None = None) -> ctypes.CDLL:
         lib = ctypes.CDLL(str(lib_path), mode=ctypes.RTLD_LOCAL)
         lib.tilemix_quant_per_block_int8.argtypes = [ctypes.POINTER(QuantParams), _vp]
         lib.tilemix_quant_per_block_int8.restype = ctypes.c_int
+        lib.tilemix_quant_per_block_int8_many.argtypes = [ctypes.POINTER(QuantParams), _i32, _i32, _vp]
+        lib.tilemix_quant_per_block_int8_many.restype = ctypes.c_int
         lib.tilemix_attn_fwd.argtypes = [ctypes.POINTER(AttnParams), _vp]
         lib.tilemix_attn_fwd.restype = ctypes.c_int
         lib.tilemix_attn_fwd_debug.argtypes = [ctypes.POINTER(AttnParams), _vp, _vp, _i64, _i64, _vp]
@@ -190,6 +193,14 @@ def quant_per_block_int8(params: QuantParams, device: torch.device) -> None:
     lib = load_library()
     with torch.cuda.device(device):
         _check(lib.tilemix_quant_per_block_int8(ctypes.byref(params), current_stream(device)), lib)
+
+
+def quant_per_block_int8_many(params: ctypes.Array, device: torch.device, uniform_seqlen: int = 0) -> None:
+    """``params``: an array of one to three ``QuantParams`` that share the batch (one launch)."""
+    lib = load_library()
+    with torch.cuda.device(device):
+        _check(lib.tilemix_quant_per_block_int8_many(params, len(params), uniform_seqlen,
+                                                      current_stream(device)), lib)
 
 
 def attn_fwd(params: AttnParams, device: torch.device) -> None:

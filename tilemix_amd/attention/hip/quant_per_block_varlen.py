@@ -9,11 +9,12 @@ attention/triton/quant_per_block_varlen.py:
   BLKQ=128, BLKK=64, sm_scale=None)`` (reference :78-106).
 
 The device kernel computes the scale-row prefix itself, so the internal
-``quantize_blocks`` used by the attention entry needs no device->host copy.
-The public ``per_block_int8_single`` still returns a scale tensor with exactly
-``cu_seqlens_x_scale[-1]`` rows, which needs the row count on the host: it is
+``quantize_many`` used by the attention entry needs no device->host copy, and it
+takes Q, K and V in one launch.
+The public functions still return scale tensors with exactly
+``cu_seqlens_x_scale[-1]`` rows, which needs the row counts on the host: they are
 taken from ``cu_seqlens_x`` directly when that lives on the CPU, otherwise read
-back once (the reference reads it back too, :62-63).
+back in one copy per call (the reference reads them back too, :62-63).
 """
 from __future__ import annotations
 
@@ -39,6 +40,31 @@ def _prepare_input(x: torch.Tensor) -> torch.Tensor:
     return x
 
 
+def _outputs(p: _native.QuantParams, x: torch.Tensor, cu: torch.Tensor, max_seqlen, blk, sm_scale, half_scales: bool,
+             cu_scale_ptr: int):
+    """Allocate one tensor's codes and scales and describe its quantisation in ``p``."""
+    device, heads, dim, batch = x.device, x.shape[1], x.shape[2], cu.numel() - 1
+    if dim % 8:
+        raise ValueError(f"head_dim must be a multiple of 8, got {dim}")
+    cap = _scale_capacity(x.shape[0], batch, blk)
+    codes = torch.empty(x.shape, dtype=torch.int8, device=device)
+    scale = torch.empty((cap, heads), dtype=torch.float32, device=device)
+    scale16 = torch.empty((cap, heads), dtype=torch.float16, device=device) if half_scales else None
+    p.input = x.data_ptr()
+    p.output = codes.data_ptr()
+    p.scale = scale.data_ptr()
+    p.scale_half = scale16.data_ptr() if scale16 is not None else None
+    p.cu_seqlens = cu.data_ptr()
+    p.cu_seqlens_scale = cu_scale_ptr
+    p.stride_in_token, p.stride_in_head = x.stride(0), x.stride(1)
+    p.stride_out_token, p.stride_out_head = codes.stride(0), codes.stride(1)
+    p.scale_rows_capacity = cap
+    p.sm_scale = float(sm_scale)
+    p.heads, p.head_dim, p.blk_tokens = heads, dim, int(blk)
+    p.batch, p.max_seqlen = batch, int(max_seqlen)
+    return codes, scale, scale16
+
+
 def quantize_blocks(x: torch.Tensor, cu_seqlens: torch.Tensor, max_seqlen: int, blk: int,
                     sm_scale: float = 1.0, *, half_scales: bool = False):
     """Quantise without any host synchronisation.
@@ -51,45 +77,59 @@ def quantize_blocks(x: torch.Tensor, cu_seqlens: torch.Tensor, max_seqlen: int, 
     device = x.device
     cu = cu_seqlens.to(device=device, dtype=torch.int32).contiguous()
     batch = cu.numel() - 1
-    heads, dim = x.shape[1], x.shape[2]
-    if dim % 8:
-        raise ValueError(f"head_dim must be a multiple of 8, got {dim}")
-    cap = _scale_capacity(x.shape[0], batch, blk)
-    codes = torch.empty(x.shape, dtype=torch.int8, device=device)
-    scale = torch.empty((cap, heads), dtype=torch.float32, device=device)
-    scale16 = torch.empty((cap, heads), dtype=torch.float16, device=device) if half_scales else None
     cu_scale = torch.empty(batch + 1, dtype=torch.int32, device=device)
+    p = _native.QuantParams()
+    codes, scale, scale16 = _outputs(p, x, cu, max_seqlen, blk, sm_scale, half_scales, cu_scale.data_ptr())
     if batch > 0:
-        p = _native.QuantParams()
-        p.input = x.data_ptr()
-        p.output = codes.data_ptr()
-        p.scale = scale.data_ptr()
-        p.scale_half = scale16.data_ptr() if scale16 is not None else None
-        p.cu_seqlens = cu.data_ptr()
-        p.cu_seqlens_scale = cu_scale.data_ptr()
-        p.stride_in_token, p.stride_in_head = x.stride(0), x.stride(1)
-        p.stride_out_token, p.stride_out_head = codes.stride(0), codes.stride(1)
-        p.scale_rows_capacity = cap
-        p.sm_scale = float(sm_scale)
-        p.heads, p.head_dim, p.blk_tokens = heads, dim, int(blk)
-        p.batch, p.max_seqlen = batch, int(max_seqlen)
         _native.quant_per_block_int8(p, device)
     else:
         cu_scale.zero_()
     return codes, scale, scale16, cu_scale
 
 
+def quantize_many(items, *, half_scales: bool = False):
+    """``quantize_blocks`` of two or three tensors ``(x, cu_seqlens, max_seqlen, blk, sm_scale)``
+    in one launch: the list of ``(codes, scale, scale16 | None)`` and the scale-row prefixes
+    int32 [len(items), B+1] (a list of them where the batches or devices differ: one
+    launch each then)."""
+    prepared = []
+    for x, cu_seqlens, *rest in items:
+        x = _prepare_input(x)
+        prepared.append((x, cu_seqlens.to(device=x.device, dtype=torch.int32).contiguous(), *rest))
+    device, entries = prepared[0][0].device, prepared[0][1].numel()
+    if any(x.device != device or cu.numel() != entries for x, cu, *_ in prepared[1:]):
+        done = [quantize_blocks(*item, half_scales=half_scales) for item in prepared]
+        return [r[:3] for r in done], [r[3] for r in done]
+    cu_scales = torch.empty((len(prepared), entries), dtype=torch.int32, device=device)
+    params = (_native.QuantParams * len(prepared))()
+    results = [_outputs(p, *item, half_scales, cu_scales.data_ptr() + 4 * i * entries)
+               for i, (p, item) in enumerate(zip(params, prepared))]
+    if entries > 1:
+        _native.quant_per_block_int8_many(params, device)
+    else:
+        cu_scales.zero_()
+    return results, cu_scales
+
+
+def scale_rows(items, cu_scales) -> list[int]:
+    """Scale rows of each item of a ``quantize_many`` call: from its ``cu_seqlens`` where that
+    lives on the CPU, else from the prefixes the launch wrote (one copy to the host for all of
+    them; the reference reads each back, :62-63)."""
+    rows = []
+    for _, cu_seqlens, _, blk, _ in items:
+        if cu_seqlens.device.type != "cpu":
+            ends = cu_scales.cpu() if isinstance(cu_scales, torch.Tensor) else [c.cpu() for c in cu_scales]
+            return [int(c[-1]) for c in ends]
+        lens = (cu_seqlens[1:] - cu_seqlens[:-1]).to(torch.int64)
+        rows.append(int(((lens + blk - 1) // blk).sum()))
+    return rows
+
+
 @torch.no_grad()
 def per_block_int8_single(x, cu_seqlens_x, max_seqlen_x, BLK=128, sm_scale=1.0):
     """Reference attention/triton/quant_per_block_varlen.py:48-75."""
-    if cu_seqlens_x.device.type == "cpu":
-        lens = (cu_seqlens_x[1:] - cu_seqlens_x[:-1]).to(torch.int64)
-        rows = int(((lens + BLK - 1) // BLK).sum())
-    else:
-        rows = None
     codes, scale, _, cu_scale = quantize_blocks(x, cu_seqlens_x, max_seqlen_x, BLK, sm_scale)
-    if rows is None:
-        rows = int(cu_scale[-1].item())
+    [rows] = scale_rows([(x, cu_seqlens_x, max_seqlen_x, BLK, sm_scale)], [cu_scale])
     return codes, scale[:rows], cu_scale.to(torch.int64)
 
 
@@ -104,8 +144,8 @@ def per_block_int8(q, k, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
         q_sm_scale = 1.0
     else:
         q_sm_scale = sm_scale * 1.44269504
-    q_int8, q_scale, cu_seqlens_q_scale = per_block_int8_single(
-        q, cu_seqlens_q, max_seqlen_q, BLK=BLKQ, sm_scale=q_sm_scale)
-    k_int8, k_scale, cu_seqlens_k_scale = per_block_int8_single(
-        k, cu_seqlens_k, max_seqlen_k, BLK=BLKK, sm_scale=1.0)
-    return q_int8, q_scale, k_int8, k_scale, cu_seqlens_q_scale, cu_seqlens_k_scale
+    items = [(q, cu_seqlens_q, max_seqlen_q, BLKQ, q_sm_scale), (k, cu_seqlens_k, max_seqlen_k, BLKK, 1.0)]
+    [(q_int8, q_scale, _), (k_int8, k_scale, _)], cu_scales = quantize_many(items)
+    rows_q, rows_k = scale_rows(items, cu_scales)
+    return (q_int8, q_scale[:rows_q], k_int8, k_scale[:rows_k],
+            cu_scales[0].to(torch.int64), cu_scales[1].to(torch.int64))

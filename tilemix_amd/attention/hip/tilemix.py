@@ -41,8 +41,8 @@ from typing import Literal, Optional
 import torch
 
 from ... import _native
-from .quant_per_block_varlen import per_block_int8 as quant_per_block_int8
-from .quant_per_block_varlen import per_block_int8_single, quantize_blocks
+from .quant_per_block_varlen import per_block_int8 as quant_per_block_int8  # noqa: F401
+from .quant_per_block_varlen import per_block_int8_single, quantize_blocks, quantize_many, scale_rows  # noqa: F401
 
 LOG2E = 1.4426950408889634
 
@@ -59,42 +59,30 @@ SUPPORTED_BLOCK_N = (64, 128, 256)
 HEAD_DIM_MULTIPLE = 16
 
 
-def _scale_dtype(dtype: torch.dtype) -> torch.dtype:
-    if dtype == torch.float16:
-        return torch.float16
-    if dtype == torch.bfloat16:
-        return torch.bfloat16
-    return torch.float32
-
-
 @torch.no_grad()
 def quantize_qkv_for_tilemix(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
                              BLKQ: int = 128, BLKK: int = 64, sm_scale: float = None):
     """Reference attention/triton/tilemix.py:45-107 (Q, K and V quantised with sm_scale=1)."""
-    q8, sq, k8, sk, cuq, cuk = quant_per_block_int8(
-        q, k, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
-        BLKQ=BLKQ, BLKK=BLKK, sm_scale=1.0)
-    v8, sv, cuv = per_block_int8_single(v, cu_seqlens_k, max_seqlen_k, BLK=BLKK, sm_scale=1.0)
-    sdt = _scale_dtype(q.dtype)
-    return (
-        q8, sq.to(dtype=sdt).contiguous(), cuq.to(dtype=torch.int32).contiguous(),
-        k8, sk.to(dtype=sdt).contiguous(), cuk.to(dtype=torch.int32).contiguous(),
-        v8, sv.to(dtype=sdt).contiguous(), cuv.to(dtype=torch.int32).contiguous(),
-    )
+    return _quantize_for_caller([(q, cu_seqlens_q, max_seqlen_q, BLKQ, 1.0), (k, cu_seqlens_k, max_seqlen_k, BLKK, 1.0),
+                                 (v, cu_seqlens_k, max_seqlen_k, BLKK, 1.0)])
 
 
 @torch.no_grad()
 def quantize_qk_for_tilemix(q, k, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
                             BLKQ: int = 128, BLKK: int = 64, sm_scale: float = None):
     """Reference attention/triton/tilemix.py:110-156."""
-    q8, sq, k8, sk, cuq, cuk = quant_per_block_int8(
-        q, k, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
-        BLKQ=BLKQ, BLKK=BLKK, sm_scale=1.0)
-    sdt = _scale_dtype(q.dtype)
-    return (
-        q8.contiguous(), sq.to(dtype=sdt).contiguous(), cuq.to(dtype=torch.int32).contiguous(),
-        k8.contiguous(), sk.to(dtype=sdt).contiguous(), cuk.to(dtype=torch.int32).contiguous(),
-    )
+    return _quantize_for_caller([(q, cu_seqlens_q, max_seqlen_q, BLKQ, 1.0), (k, cu_seqlens_k, max_seqlen_k, BLKK, 1.0)])
+
+
+def _quantize_for_caller(items) -> tuple:
+    """(codes, scales, scale-row prefix) of each item: one launch, whose kernel writes the scales
+    in Q's dtype (fp16, the only one it takes) and the int32 prefixes, and one copy of the row
+    counts to the host."""
+    results, cu_scales = quantize_many(items, half_scales=True)
+    out = []
+    for (codes, _, scale16), cu_scale, rows in zip(results, cu_scales, scale_rows(items, cu_scales)):
+        out += [codes, scale16[:rows], cu_scale]
+    return tuple(out)
 
 
 def _quantize_for_launch(t: torch.Tensor, cu: torch.Tensor, max_seqlen: int, blk: int):
@@ -496,15 +484,20 @@ def tilemix_attention_with_quant(
             raise RuntimeError("TileMix is a GPU-only HIP kernel")
         fused = _q_in_kernel_enabled() and _q_in_kernel_supported(
             block_m, BLKQ, _routing_mode_code(normalized_mode), int8_use_fp16_v)
-        if fused:
+        if fused and int8_use_fp16_v:
             q8 = sq = cuq = None
-        else:
-            q8, sq, cuq = _quantize_for_launch(q, cu_seqlens_q, max_seqlens_q, BLKQ)
-        k8, sk, cuk = _quantize_for_launch(k, cu_seqlens_k, max_seqlens_k, BLKK)
-        if int8_use_fp16_v:
+            k8, sk, cuk = _quantize_for_launch(k, cu_seqlens_k, max_seqlens_k, BLKK)
             v8, sv, cuv = _dummy_v_quantization_metadata(v, cu_seqlens_k)
         else:
-            v8, sv, cuv = _quantize_for_launch(v, cu_seqlens_k, max_seqlens_k, BLKK)
+            items = [] if fused else [(q, cu_seqlens_q, max_seqlens_q, BLKQ, 1.0)]
+            items.append((k, cu_seqlens_k, max_seqlens_k, BLKK, 1.0))
+            if not int8_use_fp16_v:
+                items.append((v, cu_seqlens_k, max_seqlens_k, BLKK, 1.0))
+            results, cu_scales = quantize_many(items, half_scales=True)
+            done = [(codes, scale16, cu) for (codes, _, scale16), cu in zip(results, cu_scales)]
+            q8, sq, cuq = (None, None, None) if fused else done.pop(0)
+            k8, sk, cuk = done.pop(0)
+            v8, sv, cuv = _dummy_v_quantization_metadata(v, cu_seqlens_k) if int8_use_fp16_v else done.pop(0)
         quantized = q8, sq, cuq, k8, sk, cuk, v8, sv, cuv
 
     q8, sq, cuq, k8, sk, cuk, v8, sv, cuv = quantized

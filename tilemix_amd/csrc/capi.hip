@@ -26,7 +26,16 @@ int tilemix_quant_per_block_int8(const tilemix_quant_params* p, void* stream) {
     tmx::set_error("tilemix_quant_per_block_int8: null params");
     return TILEMIX_E_INVALID;
   }
-  return tmx::launch_quant(*p, static_cast<hipStream_t>(stream));
+  return tmx::launch_quant(p, 1, 0, static_cast<hipStream_t>(stream));
+}
+
+int tilemix_quant_per_block_int8_many(const tilemix_quant_params* p, int32_t count, int32_t uniform_seqlen,
+                                      void* stream) {
+  if (p == nullptr) {
+    tmx::set_error("tilemix_quant_per_block_int8_many: null params");
+    return TILEMIX_E_INVALID;
+  }
+  return tmx::launch_quant(p, count, uniform_seqlen, static_cast<hipStream_t>(stream));
 }
 
 int tilemix_attn_fwd(const tilemix_attn_params* p, void* stream) {

@@ -8,20 +8,36 @@
 // plus the host-side scale bookkeeping of per_block_int8_single (:55-63),
 // done on the device so no device->host copy is needed to size the output.
 //
-// One workgroup owns one (block, head, sequence).  Blocks of up to
-// kRegChunks * 256 eight-element chunks (BLK * D <= 16384: every Q/K block of
-// the hot path) are read from HBM once and held in registers between the max
+// One workgroup owns one (tensor, sequence, block, head).  Up to kQuantMany tensors
+// (K and V, or Q, K and V of one call) go out in one launch.  Blocks of up to
+// kRegRows row groups (BLK * D <= 16384 for the usual widths: every Q/K/V block
+// of the hot path) are read from HBM once and held in registers between the max
 // pass and the code pass; larger blocks are streamed twice.
+//
+// What bounds it: HBM (2 bytes read, 1 written per element), closely followed by
+// VALU issue, so the arithmetic is kept small: a thread's rows differ by a
+// uniform stride (no division per 16-byte chunk), the block maximum is taken on
+// packed 16-bit magnitudes, and a code costs ~7 instructions (mixed-precision
+// FMAs straight from the fp16 operand, byte permutes).  Heads are the fastest
+// block index, so the workgroups in flight read neighbouring 256-byte rows.
+// Against a kernel with a 32-bit division per chunk, fp32 maxima reduced through
+// LDS, the scale-row prefix (and its barrier) before the loads, and ~12 instructions
+// per code: K of 8 x 4096 x 8 heads x 128 25.0 -> 18.5 us (5.5 TB/s), Q of 8 x 4096 x 24
+// x 128 65 -> 49 us (6.1 TB/s), K of 8 x 2048 13.6 -> 10.7 us, of 1 x 1000 5.5 -> 4.1 us.
 #include "attn_common.h"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace tmx {
 
 namespace {
 
 constexpr int kQuantThreads = 256;
-constexpr int kRegChunks = 8;
+constexpr int kRegRows = 8;    // row groups a thread holds in registers
+constexpr int kQuantMany = 3;  // tensors per launch
 
-struct QuantKArgs {
+struct QuantTensor {
   const f16* in;
   int8_t* out;
   float* scale;
@@ -31,12 +47,45 @@ struct QuantKArgs {
   int64_t si_t, si_h, so_t, so_h;
   int64_t capacity;
   float sm_scale;
-  int heads, d, blk, batch;
+  int heads, d, blk;
+  int first;  // first workgroup of this tensor within a sequence's
 };
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+struct QuantKArgs {
+  QuantTensor t[kQuantMany];
+  int count;
+  int uni;  // > 0: every sequence has this many tokens (cu is not read)
+};
+
+__device__ __forceinline__ uint32_t pk_max_u16(uint32_t x, uint32_t y) {
+  uint32_t r;
+  asm("v_pk_max_u16 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+  return r;
+}
+
+// fp32(h) - q0 * s with one rounding, for the low / high fp16 half of h2.
+__device__ __forceinline__ float rem_lo(uint32_t h2, float q0, float s) {
+  float r;
+  asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel_hi:[0,0,1]" : "=v"(r) : "v"(q0), "v"(s), "v"(h2));
+  return r;
+}
+__device__ __forceinline__ float rem_hi(uint32_t h2, float q0, float s) {
+  float r;
+  asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r) : "v"(q0), "v"(s), "v"(h2));
+  return r;
+}
+
+// Maximum over the wave (every lane gets it): lanes l ^ 32 and l ^ 16 by
+// permlane swaps, the rest of a 16-lane row by DPP moves.
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  const auto p = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  v = max((uint32_t)p[0], (uint32_t)p[1]);
+  const auto q = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = max((uint32_t)q[0], (uint32_t)q[1]);
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false));  // row_ror 8
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false));  // row_ror 4
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, false));   // quad_perm 2 3 0 1
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, false));   // quad_perm 1 0 3 2
   return v;
 }
 
@@ -46,121 +95,184 @@ __device__ __forceinline__ int wave_sum_i(int v) {
   return v;
 }
 
-__global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(const QuantKArgs a) {
-  __shared__ float red_f[kQuantThreads / 64];
-  __shared__ int red_i[kQuantThreads / 64];
-  const int blk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+// Four codes to bytes of one word.
+__device__ __forceinline__ uint32_t pack4(const int* c) {
+  return __builtin_amdgcn_perm((uint32_t)c[1], (uint32_t)c[0], 0x0c0c0400u) |
+         __builtin_amdgcn_perm((uint32_t)c[3], (uint32_t)c[2], 0x04000c0cu);
+}
+
+__global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(const QuantKArgs args) {
+  __shared__ uint32_t red[kQuantThreads / 64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int id = blockIdx.x;
+  QuantTensor a = args.t[0];
+  if (args.count > 1 && id >= args.t[1].first) a = args.t[1];
+  if (args.count > 2 && id >= args.t[2].first) a = args.t[2];
+  const int uni = args.uni;
+  const int t = id - a.first;
+  const int blk = t / a.heads, h = t - blk * a.heads;
+  const int b = blockIdx.y;
 
-  // Scale-row base of sequence b: sum over earlier sequences of ceil(L/blk).
-  int part = 0;
-  for (int bb = tid; bb < b; bb += kQuantThreads) {
-    const int len = a.cu[bb + 1] - a.cu[bb];
-    part += (len + a.blk - 1) / a.blk;
+  const int start = uni > 0 ? b * uni : a.cu[b];
+  const int len = uni > 0 ? uni : a.cu[b + 1] - start;
+  const int rows = min(a.blk, len - blk * a.blk);  // <= 0: no such block in this sequence
+
+  // Scale-row base of sequence b (the sum of ceil(L / blk) over the earlier
+  // ones), needed by wave 0 only: it stores the scale.  Called after the block's
+  // loads have gone out.
+  auto scale_base = [&]() -> int {
+    if (uni > 0) return b * ((uni + a.blk - 1) / a.blk);
+    int part = 0;
+    for (int bb = lane; bb < b; bb += 64) part += (a.cu[bb + 1] - a.cu[bb] + a.blk - 1) / a.blk;
+    return wave_sum_i(part);
+  };
+  auto publish = [&](int base) {
+    if (blk == 0 && h == 0 && tid == 0 && a.cu_scale != nullptr) {
+      a.cu_scale[b + 1] = base + (len + a.blk - 1) / a.blk;
+      if (b == 0) a.cu_scale[0] = 0;
+    }
+  };
+  if (rows <= 0) {
+    if (blk == 0 && h == 0 && wave == 0) publish(scale_base());
+    return;
   }
-  part = wave_sum_i(part);
-  if (lane == 0) red_i[wave] = part;
-  __syncthreads();
-  int base = 0;
-#pragma unroll
-  for (int w = 0; w < kQuantThreads / 64; ++w) base += red_i[w];
 
-  const int start = a.cu[b];
-  const int len = a.cu[b + 1] - start;
-  if (blk == 0 && h == 0 && tid == 0 && a.cu_scale != nullptr) {
-    a.cu_scale[b + 1] = base + (len + a.blk - 1) / a.blk;
-    if (b == 0) a.cu_scale[0] = 0;
-  }
-  if (blk * a.blk >= len) return;
-
-  const int rows = min(a.blk, len - blk * a.blk);
-  const int cpr = a.d >> 3;  // 8-element chunks per row
-  const int chunks = rows * cpr;
+  const int cpr = a.d >> 3;                // 8-element chunks per row
+  const int rpi = kQuantThreads / cpr;     // rows the workgroup reads per step
+  const int r0 = tid / cpr, col = (tid - r0 * cpr) << 3;
+  const bool used = r0 < rpi;              // cpr need not divide the workgroup
+  const int groups = (rows + rpi - 1) / rpi;
   const int64_t tok0 = (int64_t)start + (int64_t)blk * a.blk;
-  const f16* in = a.in + tok0 * a.si_t + (int64_t)h * a.si_h;
-  int8_t* out = a.out + tok0 * a.so_t + (int64_t)h * a.so_h;
+  const f16* in = a.in + (tok0 + r0) * a.si_t + (int64_t)h * a.si_h + col;
+  int8_t* out = a.out + (tok0 + r0) * a.so_t + (int64_t)h * a.so_h + col;
+  const int64_t in_step = (int64_t)rpi * a.si_t, out_step = (int64_t)rpi * a.so_t;
 
   const float sm = a.sm_scale;
   // sm_scale == 1 (the hot path: quantize_q(k)_for_tilemix): the quotient is
-  // taken from an IEEE reciprocal with one correction step, equal to the IEEE
-  // division on the whole fp16 domain; other scales divide directly.
+  // taken from an IEEE reciprocal with one correction step (div_by_recip),
+  // equal to the IEEE division on the whole fp16 domain; other scales divide
+  // directly.
   const bool unit_scale = sm == 1.0f;
-  auto encode = [&](const f16x8& x, float s, float rs, int r, int col) {
-    uint32_t w0 = 0, w1 = 0;
+  auto encode = [&](const u32x4& x, float s, float rs, int8_t* dst) {
+    int c[8];
+    if (unit_scale) {
+      // rs is 0 for an all-zero block, whose codes then come out as 0.
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float t = unit_scale ? div_by_recip((float)x[e], s, rs) : ((float)x[e] * sm) / s;
-      t += (t >= 0.0f) ? 0.5f : -0.5f;
-      // An all-zero block gives 0/0; its codes are defined as 0.
-      const int code = (s == 0.0f) ? 0 : (int)t;
-      const uint32_t byte = (uint32_t)(code & 0xff);
-      if (e < 4) w0 |= byte << (8 * e);
-      else w1 |= byte << (8 * (e - 4));
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t h2 = x[e >> 1];
+        const float q0 = (e & 1) ? mul_hi(h2, rs) : mul_lo(h2, rs);
+        const float rem = (e & 1) ? rem_hi(h2, q0, s) : rem_lo(h2, q0, s);
+        float v = __builtin_fmaf(rem, rs, q0);
+        // v + (v >= 0 ? 0.5 : -0.5); they differ only at v = -0, where both
+        // truncate to code 0.
+        v += __builtin_copysignf(0.5f, v);
+        c[e] = (int)v;
+      }
+    } else {
+      const f16x8 xv = __builtin_bit_cast(f16x8, x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float v = ((float)xv[e] * sm) / s;
+        v += (v >= 0.0f) ? 0.5f : -0.5f;
+        c[e] = (s == 0.0f) ? 0 : (int)v;
+      }
     }
-    *reinterpret_cast<uint2*>(out + (int64_t)r * a.so_t + col) = make_uint2(w0, w1);
+    *reinterpret_cast<uint2*>(dst) = make_uint2(pack4(c), pack4(c + 4));
   };
-  auto block_max = [&](float amax) {
-    amax = wave_max(amax);
-    if (lane == 0) red_f[wave] = amax;
+  // max|x * sm| over the block from the lane's largest magnitude (packed 16-bit
+  // patterns without their signs order like the values; RN(x * sm) is monotonic
+  // in |x|).  The maximum ignores NaNs, whose patterns lie above infinity's: a
+  // block that holds one takes its maximum again from the values below.
+  auto block_max = [&](uint32_t m2) -> uint32_t {
+    const uint32_t m = wave_max_u32(max(m2 & 0xffffu, m2 >> 16));
     __syncthreads();
-    amax = red_f[0];
+    if (lane == 0) red[wave] = m;
+    __syncthreads();
+    uint32_t r = red[0];
 #pragma unroll
-    for (int w = 1; w < kQuantThreads / 64; ++w) amax = fmaxf(amax, red_f[w]);
-    return amax;
+    for (int w = 1; w < kQuantThreads / 64; ++w) r = max(r, red[w]);
+    return r;
+  };
+  constexpr uint32_t kInf = 0x7c00u;
+  auto magnitudes = [](const u32x4& x, uint32_t m2) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m2 = pk_max_u16(m2, x[e] & 0x7fff7fffu);
+    return m2;
+  };
+  auto finite_magnitudes = [&](const u32x4& x, uint32_t m2) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t lo = x[e] & 0x7fffu, hi = (x[e] >> 16) & 0x7fffu;
+      m2 = pk_max_u16(m2, (lo > kInf ? 0u : lo) | ((hi > kInf ? 0u : hi) << 16));
+    }
+    return m2;
+  };
+  auto scale_of = [&](uint32_t m) -> float {
+    const float amax = fmaxf(0.0f, fabsf((float)__builtin_bit_cast(f16, (uint16_t)m) * sm));
+    return amax / 127.0f;  // IEEE division (no fast-math in this build)
+  };
+  auto finish = [&](float s, int base) {
+    if (tid == 0) {
+      const int64_t row = (int64_t)base + blk;
+      if (row < a.capacity) {
+        a.scale[row * a.heads + h] = s;
+        if (a.scale_half != nullptr) a.scale_half[row * a.heads + h] = (f16)s;
+      }
+    }
+    publish(base);
   };
 
-  float s;
-  if (chunks <= kRegChunks * kQuantThreads) {
-    f16x8 xs[kRegChunks];
-    float amax = 0.0f;
+  auto in_registers = [&](auto nreg) {
+    constexpr int kN = decltype(nreg)::value;
+    u32x4 xs[kN];
+    uint32_t m2 = 0;
 #pragma unroll
-    for (int i = 0; i < kRegChunks; ++i) {
-      const int c = tid + i * kQuantThreads;
-      if (c < chunks) {
-        const int r = c / cpr, col = (c - r * cpr) << 3;
-        xs[i] = *reinterpret_cast<const f16x8*>(in + (int64_t)r * a.si_t + col);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf((float)xs[i][e] * sm));
-      }
+    for (int i = 0; i < kN; ++i) {
+      xs[i] = (u32x4){};
+      if (used && r0 + i * rpi < rows) xs[i] = *reinterpret_cast<const u32x4*>(in + i * in_step);
     }
-    s = block_max(amax) / 127.0f;  // IEEE division (no fast-math in this build)
-    const float rs = 1.0f / s;
+    const int base = wave == 0 ? scale_base() : 0;
 #pragma unroll
-    for (int i = 0; i < kRegChunks; ++i) {
-      const int c = tid + i * kQuantThreads;
-      if (c < chunks) {
-        const int r = c / cpr, col = (c - r * cpr) << 3;
-        encode(xs[i], s, rs, r, col);
-      }
+    for (int i = 0; i < kN; ++i) m2 = magnitudes(xs[i], m2);
+    uint32_t m = block_max(m2);
+    if (m > kInf) {
+      m2 = 0;
+#pragma unroll
+      for (int i = 0; i < kN; ++i) m2 = finite_magnitudes(xs[i], m2);
+      m = block_max(m2);
     }
+    const float s = scale_of(m);
+    const float rs = s == 0.0f ? 0.0f : 1.0f / s;
+#pragma unroll
+    for (int i = 0; i < kN; ++i)
+      if (used && r0 + i * rpi < rows) encode(xs[i], s, rs, out + i * out_step);
+    finish(s, base);
+  };
+  if (groups <= kRegRows / 2) {
+    in_registers(std::integral_constant<int, kRegRows / 2>{});
+  } else if (groups <= kRegRows) {
+    in_registers(std::integral_constant<int, kRegRows>{});
   } else {
-    float amax = 0.0f;
-    for (int c = tid; c < chunks; c += kQuantThreads) {
-      const int r = c / cpr, col = (c - r * cpr) << 3;
-      const f16x8 x = *reinterpret_cast<const f16x8*>(in + (int64_t)r * a.si_t + col);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf((float)x[e] * sm));
+    uint32_t m2 = 0;
+    for (int i = 0; used && r0 + i * rpi < rows; ++i)
+      m2 = magnitudes(*reinterpret_cast<const u32x4*>(in + i * in_step), m2);
+    uint32_t m = block_max(m2);
+    if (m > kInf) {
+      m2 = 0;
+      for (int i = 0; used && r0 + i * rpi < rows; ++i)
+        m2 = finite_magnitudes(*reinterpret_cast<const u32x4*>(in + i * in_step), m2);
+      m = block_max(m2);
     }
-    s = block_max(amax) / 127.0f;
-    const float rs = 1.0f / s;
-    for (int c = tid; c < chunks; c += kQuantThreads) {
-      const int r = c / cpr, col = (c - r * cpr) << 3;
-      encode(*reinterpret_cast<const f16x8*>(in + (int64_t)r * a.si_t + col), s, rs, r, col);
-    }
-  }
-  if (tid == 0) {
-    const int64_t row = (int64_t)base + blk;
-    if (row < a.capacity) {
-      a.scale[row * a.heads + h] = s;
-      if (a.scale_half != nullptr) a.scale_half[row * a.heads + h] = (f16)s;
-    }
+    const float s = scale_of(m);
+    const float rs = s == 0.0f ? 0.0f : 1.0f / s;
+    for (int i = 0; used && r0 + i * rpi < rows; ++i)
+      encode(*reinterpret_cast<const u32x4*>(in + i * in_step), s, rs, out + i * out_step);
+    finish(s, wave == 0 ? scale_base() : 0);
   }
 }
 
-}  // namespace
-
-int launch_quant(const tilemix_quant_params& p, hipStream_t stream) {
-  if (!p.input || !p.output || !p.scale || !p.cu_seqlens) {
+int check_quant(const tilemix_quant_params& p, bool uniform) {
+  if (!p.input || !p.output || !p.scale || (!uniform && !p.cu_seqlens)) {
     set_error("tilemix_quant_per_block_int8: null tensor pointer");
     return TILEMIX_E_INVALID;
   }
@@ -180,28 +292,60 @@ int launch_quant(const tilemix_quant_params& p, hipStream_t stream) {
               "elements; output 8-byte aligned with strides multiple of 8");
     return TILEMIX_E_INVALID;
   }
-  if (p.batch == 0) return TILEMIX_OK;
-  const int nblk = (p.max_seqlen + p.blk_tokens - 1) / p.blk_tokens;
+  return TILEMIX_OK;
+}
+
+}  // namespace
+
+int launch_quant(const tilemix_quant_params* ps, int count, int uniform_seqlen, hipStream_t stream) {
+  if (count < 1 || count > kQuantMany || uniform_seqlen < 0) {
+    set_error("tilemix_quant_per_block_int8: 1 to %d tensors and a non-negative uniform length, got %d and %d",
+              kQuantMany, count, uniform_seqlen);
+    return TILEMIX_E_INVALID;
+  }
   QuantKArgs a;
-  a.in = static_cast<const f16*>(p.input);
-  a.out = p.output;
-  a.scale = p.scale;
-  a.scale_half = static_cast<f16*>(p.scale_half);
-  a.cu = p.cu_seqlens;
-  a.cu_scale = p.cu_seqlens_scale;
-  a.si_t = p.stride_in_token;
-  a.si_h = p.stride_in_head;
-  a.so_t = p.stride_out_token;
-  a.so_h = p.stride_out_head;
-  a.capacity = p.scale_rows_capacity;
-  a.sm_scale = p.sm_scale;
-  a.heads = p.heads;
-  a.d = p.head_dim;
-  a.blk = p.blk_tokens;
-  a.batch = p.batch;
-  // With no tokens, one block per sequence still publishes cu_seqlens_scale.
-  dim3 grid(nblk > 0 ? nblk : 1, p.heads, p.batch);
-  hipLaunchKernelGGL(quant_per_block_int8_kernel, grid, dim3(kQuantThreads), 0, stream, a);
+  a.count = 0;
+  a.uni = uniform_seqlen;
+  int64_t total = 0;
+  for (int i = 0; i < count; ++i) {
+    const tilemix_quant_params& p = ps[i];
+    const int status = check_quant(p, uniform_seqlen > 0);
+    if (status != TILEMIX_OK) return status;
+    if (p.batch != ps[0].batch) {
+      set_error("tilemix_quant_per_block_int8: the tensors of one launch share the batch, got %d and %d",
+                ps[0].batch, p.batch);
+      return TILEMIX_E_INVALID;
+    }
+    const int max_seqlen = uniform_seqlen > 0 ? uniform_seqlen : p.max_seqlen;
+    // With no tokens, one block per sequence still publishes cu_seqlens_scale.
+    const int64_t nblk = std::max<int64_t>(1, ((int64_t)max_seqlen + p.blk_tokens - 1) / p.blk_tokens);
+    QuantTensor& t = a.t[a.count++];
+    t.in = static_cast<const f16*>(p.input);
+    t.out = p.output;
+    t.scale = p.scale;
+    t.scale_half = static_cast<f16*>(p.scale_half);
+    t.cu = p.cu_seqlens;
+    t.cu_scale = p.cu_seqlens_scale;
+    t.si_t = p.stride_in_token;
+    t.si_h = p.stride_in_head;
+    t.so_t = p.stride_out_token;
+    t.so_h = p.stride_out_head;
+    t.capacity = p.scale_rows_capacity;
+    t.sm_scale = p.sm_scale;
+    t.heads = p.heads;
+    t.d = p.head_dim;
+    t.blk = p.blk_tokens;
+    t.first = (int)total;
+    total += nblk * p.heads;
+    if (total > INT32_MAX) {
+      set_error("tilemix_quant_per_block_int8: too many blocks (%lld)", (long long)total);
+      return TILEMIX_E_INVALID;
+    }
+  }
+  if (ps[0].batch == 0) return TILEMIX_OK;
+  for (int i = a.count; i < kQuantMany; ++i) a.t[i] = a.t[0];
+  hipLaunchKernelGGL(quant_per_block_int8_kernel, dim3((unsigned)total, (unsigned)ps[0].batch),
+                     dim3(kQuantThreads), 0, stream, a);
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) {
     set_error("tilemix_quant_per_block_int8: launch failed: %s", hipGetErrorString(err));
