@@ -1,0 +1,67 @@
+"""Prefill helper kernels at the edges of their dispatch: RMSNorm widths on both sides
+of every per-lane chunk count, rotary head dims around the workgroup shapes (head slots,
+tokens per workgroup, the element-wise limit) with ragged token and head counts, and
+SiLU * up on every fp16 gate.  Bars as in test_gpu_prefill_helpers.py."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import prefill_oracle as PO
+from test_gpu_prefill_helpers import _rope_inputs, _within_ulps
+from tilemix_amd.models import tilemix_llama as TL
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("cols", [8, 512, 1024, 1032, 2048, 2056, 3072, 3075, 3080, 4096, 4104, 8184, 8192, 8200])
+@pytest.mark.parametrize("rows", [1, 6])
+def test_rms_norm_chunk_counts(device, cols, rows):
+    g = torch.Generator().manual_seed(cols + rows)
+    x = torch.randn(rows, cols, generator=g).half()
+    w = (torch.randn(cols, generator=g) * 0.3 + 1.0).half()
+    ok, frac = _within_ulps(TL.rms_norm(x.to(device), w.to(device), 1e-5), PO.rms_norm(x, w, 1e-5), 2)
+    assert ok and frac <= max(0.01, 1.5 / (rows * cols)), frac
+
+
+def test_rms_norm_row_stride_aligned_and_not(device):
+    """Rows of 3072 columns inside wider buffers: a stride that keeps 16-byte alignment and one that does not."""
+    g = torch.Generator().manual_seed(5)
+    w = (torch.randn(3072, generator=g) * 0.3 + 1.0).half()
+    for width in (3088, 3076):
+        base = torch.randn(9, width, generator=g).half()
+        got = TL.rms_norm(base.to(device)[:, :3072], w.to(device), 1e-5)
+        ok, frac = _within_ulps(got, PO.rms_norm(base[:, :3072], w, 1e-5), 2)
+        assert ok and frac <= 0.01, (width, frac)
+
+
+@pytest.mark.parametrize("b,hq,hk,t,d", [
+    (1, 17, 1, 1, 16),      # one chunk pair per row, one head past the 16 slots
+    (2, 33, 16, 5, 64),     # three passes over the head slots
+    (3, 5, 5, 7, 80),       # pairs that do not divide the workgroup
+    (1, 16, 15, 3, 256),    # one token per workgroup
+    (1, 20, 2, 3, 272),     # fewer than 16 head slots
+    (1, 2, 1, 2, 4096),     # one head slot, one token
+    (1, 2, 1, 2, 4112),     # past the vector path
+])
+def test_rotary_shapes_bitexact(device, b, hq, hk, t, d):
+    q, k, cos, sin = _rope_inputs(b, hq, hk, t, d, b, seed=d + t, device=device)
+    wq, wk = PO.rotary_token_major(q, k, cos, sin)
+    gq, gk = TL.rotary_token_major(q.to(device), k.to(device), cos.to(device), sin.to(device))
+    assert torch.equal(gq.cpu(), wq) and torch.equal(gk.cpu(), wk)
+    hm_q, hm_k = (x.contiguous().to(device) for x in (q, k))  # head-major inputs
+    gq, gk = TL.rotary_token_major(hm_q, hm_k, cos.to(device), sin.to(device))
+    assert torch.equal(gq.cpu(), wq) and torch.equal(gk.cpu(), wk)
+
+
+@pytest.mark.parametrize("up", [1.0, -0.37])
+def test_silu_mul_every_gate(device, up):
+    """All 65536 fp16 gates: infinities and NaNs as in the formula, finite results within one ulp."""
+    gate = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    ups = torch.full_like(gate, up)
+    got, want = TL.silu_mul(gate.to(device), ups.to(device)).cpu(), PO.silu_mul(gate, ups)
+    finite = torch.isfinite(want)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)]) and torch.isfinite(got[finite]).all()
+    ok, frac = _within_ulps(got[finite], want[finite], 1)
+    assert ok and frac <= 1e-3, frac

@@ -19,14 +19,42 @@ __device__ __forceinline__ float keep32(float x) {
   return x;
 }
 
+// RN(h * s) of the low / high fp16 half of h2 (one rounding; the addend -0 keeps
+// the sign of a zero product).
+__device__ __forceinline__ float mul_half(uint32_t h2, float s, bool high) {
+  float r;
+  if (high)
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h2), "v"(s), "v"(-0.0f));
+  else
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h2), "v"(s), "v"(-0.0f));
+  return r;
+}
+// acc + h * h of the low / high fp16 half of h2 in fp32.
+__device__ __forceinline__ float add_square(uint32_t h2, float acc, bool high) {
+  float r;
+  if (high)
+    asm("v_fma_mix_f32 %0, %1, %1, %2 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(r) : "v"(h2), "v"(acc));
+  else
+    asm("v_fma_mix_f32 %0, %1, %1, %2 op_sel_hi:[1,1,0]" : "=v"(r) : "v"(h2), "v"(acc));
+  return r;
+}
+
 // ---- RMSNorm (reference :718-797) ------------------------------------------
 // The sum of squares adds separately rounded products (the reference's
-// reduction is built without FMA contraction), in this kernel's own order.
-// One wave per row; rows of up to kNormChunks * 64 eight-element chunks
-// (cols <= 8192) stay in registers between the sum of squares and the output
-// pass, longer rows are read twice.
+// reduction is built without FMA contraction; the square of an fp16 value is
+// exact in fp32, so one mixed-precision FMA per value gives the same sum), in
+// this kernel's own order.  One wave per row; rows of up to 16 * 64 eight-element
+// chunks (cols <= 8192) stay in registers between the sum of squares and the
+// output pass, longer rows are read twice.
+//
+// Bound by HBM (4 bytes per value).  The kernel is instantiated per number of
+// chunks a lane holds (NCH), so that a row takes only the registers it needs and
+// more waves keep loads in flight, and the fp32 work is two instructions per
+// value (an fp16 product of two fp16 values is their exact fp32 product rounded
+// once).  Against one instantiation for every width with fp32 multiplies and adds
+// (us): 32768 x 3072 88 -> 78 (5.2 TB/s, a large copy's rate), 8192 x 2048 15.6 -> 12.8,
+// 2048 x 3072 7.8 -> 7.0, 4096 x 8192 23.5 -> 22.9.
 constexpr int kNormWaves = 4;
-constexpr int kNormChunks = 16;
 
 struct NormArgs {
   const f16* x;
@@ -48,6 +76,9 @@ __device__ __forceinline__ f16 norm_one(float x, float rs, f16 w) {
   return (f16)((float)w * (float)hn);        // fp16(fp32(w) * fp32(hn))
 }
 
+// NCH: 8-element chunks a lane holds; 0 = rows longer than 16 chunks a lane, or
+// not 16-byte aligned (element by element).
+template <int NCH>
 __global__ void __launch_bounds__(kNormWaves * 64) rmsnorm_kernel(const NormArgs a) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * kNormWaves + (threadIdx.x >> 6);
@@ -56,32 +87,31 @@ __global__ void __launch_bounds__(kNormWaves * 64) rmsnorm_kernel(const NormArgs
   f16* orow = a.out + row * a.so;
   const int chunks = a.cols >> 3;          // full 8-element chunks
   const int tail0 = chunks << 3;           // first element of the ragged tail
-  const bool vec = ((reinterpret_cast<uintptr_t>(xr) | reinterpret_cast<uintptr_t>(orow) |
-                     reinterpret_cast<uintptr_t>(a.w)) & 15) == 0;
   float ss = 0.0f;
-  if (vec && chunks <= kNormChunks * 64) {
-    f16x8 xv[kNormChunks];
+  if constexpr (NCH > 0) {
+    u32x4 xv[NCH];
 #pragma unroll
-    for (int i = 0; i < kNormChunks; ++i) {
+    for (int i = 0; i < NCH; ++i) {
       const int c = i * 64 + lane;
-      if (c < chunks) {
-        xv[i] = *reinterpret_cast<const f16x8*>(xr + c * 8);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) ss += (float)xv[i][e] * (float)xv[i][e];
-      }
+      xv[i] = (u32x4){};
+      if (c < chunks) xv[i] = *reinterpret_cast<const u32x4*>(xr + c * 8);
     }
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss = add_square(xv[i][e >> 1], ss, e & 1);
     for (int c = tail0 + lane; c < a.cols; c += 64) ss += (float)xr[c] * (float)xr[c];
     const float var = wave_sum(ss) * a.inv_cols;
     const float rs = 1.0f / sqrtf(var + a.eps);
 #pragma unroll
-    for (int i = 0; i < kNormChunks; ++i) {
+    for (int i = 0; i < NCH; ++i) {
       const int c = i * 64 + lane;
       if (c < chunks) {
         const f16x8 wv = *reinterpret_cast<const f16x8*>(a.w + c * 8);
-        f16x8 o;
+        f16x8 hn;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = norm_one((float)xv[i][e], rs, wv[e]);
-        *reinterpret_cast<f16x8*>(orow + c * 8) = o;
+        for (int e = 0; e < 8; ++e) hn[e] = (f16)mul_half(xv[i][e >> 1], rs, e & 1);
+        *reinterpret_cast<f16x8*>(orow + c * 8) = wv * hn;
       }
     }
     for (int c = tail0 + lane; c < a.cols; c += 64) orow[c] = norm_one((float)xr[c], rs, a.w[c]);
@@ -94,8 +124,15 @@ __global__ void __launch_bounds__(kNormWaves * 64) rmsnorm_kernel(const NormArgs
 }
 
 // ---- rotary (reference :808-847) -------------------------------------------
-// One thread per 8-element chunk of one (b, t, h) row; the partner chunk at
-// d' = (d + D/2) % D is loaded directly.  Output rows are token-major.
+// One thread per pair of 8-element chunks (d, d + D/2) of a (b, t, h) row: the two
+// chunks are each other's rotation partners, so a row is read once.  A thread
+// takes every 16th head (fewer slots for head_dim > 256) of its token with the
+// token's cos / sin chunks in registers.  Output rows are token-major.  Bound by
+// HBM (4 bytes per value) at large token counts, by loads in flight at small ones.
+// Against one thread per chunk that loads its partner chunk too (24 + 8 heads, head_dim
+// 128, us): 2048 tokens 10.8 -> 8.8, 2 x 1537 head-major 13.7 -> 11.9, 32768 tokens 100 ->
+// 101 (5.5 TB/s, a large copy's rate); 8192 tokens of 32 + 8 heads x 64 19.1 -> 16.7.  8 slots:
+// 8.7 / 11.5 / 104 / 16.2; 4 slots: 9.9 / 12.4 / 107 / 19.4.
 struct RotaryArgs {
   const f16* q;
   const f16* k;
@@ -104,7 +141,8 @@ struct RotaryArgs {
   f16* oq;
   f16* ok;
   int64_t qz, qh, qt, kz, kh, kt, cz, ct, sz, st;
-  int64_t rows;  // batch * tokens * (hq + hk)
+  int64_t bt;    // batch * tokens
+  int64_t rows;  // bt * (hq + hk)
   int t, hq, hk, d;
 };
 
@@ -114,38 +152,43 @@ __device__ __forceinline__ f16 rope_one(float x, float xr, float c, float s, flo
   return (f16)keep32((float)a + (float)b);
 }
 
-__global__ void __launch_bounds__(256) rotary_kernel(const RotaryArgs a) {
-  const int cpr = a.d >> 3;  // chunks per row (d % 16 == 0 on this path)
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= a.rows * cpr) return;
-  const int ch = (int)(gid % cpr);
-  int64_t r = gid / cpr;
-  const int H = a.hq + a.hk;
-  const int h = (int)(r % H);
-  r /= H;
-  const int t = (int)(r % a.t);
-  const int64_t b = r / a.t;
-  const int d0 = ch * 8;
-  const int half = a.d >> 1;
-  const int dr = d0 < half ? d0 + half : d0 - half;
-  const float sign = d0 < half ? -1.0f : 1.0f;
-  const f16* src;
-  f16* dst;
-  if (h < a.hq) {
-    src = a.q + b * a.qz + (int64_t)h * a.qh + (int64_t)t * a.qt;
-    dst = a.oq + ((b * a.t + t) * a.hq + h) * a.d;
-  } else {
-    src = a.k + b * a.kz + (int64_t)(h - a.hq) * a.kh + (int64_t)t * a.kt;
-    dst = a.ok + ((b * a.t + t) * a.hk + (h - a.hq)) * a.d;
-  }
-  const f16x8 x = *reinterpret_cast<const f16x8*>(src + d0);
-  const f16x8 xr = *reinterpret_cast<const f16x8*>(src + dr);
-  const f16x8 c = *reinterpret_cast<const f16x8*>(a.cs + b * a.cz + (int64_t)t * a.ct + d0);
-  const f16x8 s = *reinterpret_cast<const f16x8*>(a.sn + b * a.sz + (int64_t)t * a.st + d0);
+// Workgroup shape for rows of `pairs` chunk pairs: head slots per token (at most 16)
+// and tokens.
+__host__ __device__ inline int rot_heads(int pairs) { return min(16, 256 / pairs); }
+__host__ __device__ inline int rot_tokens(int pairs) { return 256 / pairs / rot_heads(pairs); }
+
+__device__ __forceinline__ f16x8 rope8(const f16x8& x, const f16x8& xr, const f16x8& c, const f16x8& s, float sign) {
   f16x8 o;
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = rope_one((float)x[e], (float)xr[e], (float)c[e], (float)s[e], sign);
-  *reinterpret_cast<f16x8*>(dst + d0) = o;
+  return o;
+}
+
+__global__ void __launch_bounds__(256) rotary_kernel(const RotaryArgs a) {
+  const int half = a.d >> 1;
+  const int cpr = half >> 3;                // chunk pairs per row (d % 16 == 0 on this path)
+  const int heads = rot_heads(cpr), tokens = rot_tokens(cpr);
+  const int slot = threadIdx.x / cpr, d0 = (threadIdx.x - slot * cpr) * 8;
+  const int tl = slot / heads, h0 = slot - tl * heads;
+  const int64_t bt = (int64_t)blockIdx.x * tokens + tl;
+  if (tl >= tokens || bt >= a.bt) return;
+  const int64_t b = bt / a.t, t = bt - b * a.t;
+  const f16* cs = a.cs + b * a.cz + t * a.ct + d0;
+  const f16* sn = a.sn + b * a.sz + t * a.st + d0;
+  const f16x8 c0 = *reinterpret_cast<const f16x8*>(cs), c1 = *reinterpret_cast<const f16x8*>(cs + half);
+  const f16x8 s0 = *reinterpret_cast<const f16x8*>(sn), s1 = *reinterpret_cast<const f16x8*>(sn + half);
+  // Heads h0, h0 + heads, ... of one tensor's n.
+  auto rotate = [&](const f16* src, f16* dst, int n, int64_t head_stride) {
+    for (int h = h0; h < n; h += heads) {
+      const f16* x = src + h * head_stride;
+      const f16x8 x0 = *reinterpret_cast<const f16x8*>(x), x1 = *reinterpret_cast<const f16x8*>(x + half);
+      f16* o = dst + (int64_t)h * a.d;
+      *reinterpret_cast<f16x8*>(o) = rope8(x0, x1, c0, s0, -1.0f);
+      *reinterpret_cast<f16x8*>(o + half) = rope8(x1, x0, c1, s1, 1.0f);
+    }
+  };
+  rotate(a.q + b * a.qz + t * a.qt + d0, a.oq + bt * a.hq * a.d + d0, a.hq, a.qh);
+  rotate(a.k + b * a.kz + t * a.kt + d0, a.ok + bt * a.hk * a.d + d0, a.hk, a.kh);
 }
 
 // Generic element-wise variant (any even head_dim, any alignment).
@@ -177,10 +220,24 @@ __global__ void __launch_bounds__(256) rotary_kernel_scalar(const RotaryArgs a) 
 }
 
 // ---- SiLU * up (reference :850-869) -----------------------------------------
+// g / den correctly rounded (den >= 1): a Newton step on the hardware reciprocal,
+// Markstein's correction of the quotient, and the fix-up instruction for
+// infinities and NaNs.  A quotient too small for its remainder to be exact lies
+// far below half of fp16's smallest value and becomes 0 either way; a denominator
+// of infinity (exp(-g) overflows) is such a case.  The full IEEE division adds
+// scaling steps for ranges that do not occur here; all 65536 gate values give the
+// same bits.  2048 x 8192: 19.5 -> 18.4 us; 32768 x 8192 is HBM-bound either way
+// (276 -> 273 us, 5.9 TB/s).
+__device__ __forceinline__ float silu_div(float g, float den) {
+  float r = __builtin_amdgcn_rcpf(den);
+  r = __builtin_fmaf(__builtin_fmaf(-den, r, 1.0f), r, r);
+  const float q = g * r;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, den, g), r, q), den, g);
+}
 __device__ __forceinline__ f16 silu_mul_one(f16 g16, f16 u16) {
   const float g = (float)g16;
-  const f16 act = (f16)keep32(g / keep32(1.0f + expf(-g)));  // IEEE division
-  return (f16)((float)act * (float)u16);
+  const f16 act = (f16)keep32(silu_div(g, keep32(1.0f + expf(-g))));
+  return act * u16;  // fp16 product: the exact fp32 product rounded once
 }
 
 __global__ void __launch_bounds__(256) silu_mul_kernel(const f16* g, const f16* u, f16* o, int64_t n) {
@@ -236,9 +293,30 @@ int launch_rmsnorm(const tilemix_rmsnorm_params& p, hipStream_t stream) {
   a.cols = p.cols;
   a.inv_cols = 1.0f / (float)p.cols;  // the mean's factor, as fp32(1/N)
   a.eps = p.eps;
-  // Rows whose start is not 16-byte aligned take the kernel's scalar branch.
-  const int64_t blocks = (p.rows + kNormWaves - 1) / kNormWaves;
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)blocks), dim3(kNormWaves * 64), 0, stream, a);
+  // Rows that are not all 16-byte aligned are read element by element.
+  const bool vec = aligned16(p.x) && aligned16(p.out) && aligned16(p.weight) &&
+                   (p.rows == 1 || ((p.stride_x | p.stride_out) & 7) == 0);
+  const int lane_chunks = vec ? (p.cols / 8 + 63) / 64 : 0;  // per lane
+  const dim3 grid((unsigned)((p.rows + kNormWaves - 1) / kNormWaves)), block(kNormWaves * 64);
+  switch (lane_chunks > 16 ? 0 : lane_chunks > 8 ? 16 : lane_chunks > 6 ? 8 : (lane_chunks + 1) / 2 * 2) {
+    case 2:
+      hipLaunchKernelGGL((rmsnorm_kernel<2>), grid, block, 0, stream, a);
+      break;
+    case 4:
+      hipLaunchKernelGGL((rmsnorm_kernel<4>), grid, block, 0, stream, a);
+      break;
+    case 6:
+      hipLaunchKernelGGL((rmsnorm_kernel<6>), grid, block, 0, stream, a);
+      break;
+    case 8:
+      hipLaunchKernelGGL((rmsnorm_kernel<8>), grid, block, 0, stream, a);
+      break;
+    case 16:
+      hipLaunchKernelGGL((rmsnorm_kernel<16>), grid, block, 0, stream, a);
+      break;
+    default:
+      hipLaunchKernelGGL((rmsnorm_kernel<0>), grid, block, 0, stream, a);
+  }
   return check_launch("tilemix_rms_norm_f16");
 }
 
@@ -274,16 +352,17 @@ int launch_rotary(const tilemix_rotary_params& p, hipStream_t stream) {
   a.hq = p.heads_q;
   a.hk = p.heads_k;
   a.d = p.head_dim;
-  a.rows = (int64_t)p.batch * p.tokens * (p.heads_q + p.heads_k);
+  a.bt = (int64_t)p.batch * p.tokens;
+  a.rows = a.bt * (p.heads_q + p.heads_k);
   if (a.rows == 0) return TILEMIX_OK;
   // 16-byte chunks need head_dim % 16 == 0 (so both halves are chunk aligned)
   // and every row start 16-byte aligned.
-  const bool vec = (p.head_dim % 16) == 0 && aligned16(p.q) && aligned16(p.k) && aligned16(p.cos) &&
+  const bool vec = (p.head_dim % 16) == 0 && p.head_dim <= 16 * 256 && aligned16(p.q) && aligned16(p.k) && aligned16(p.cos) &&
                    aligned16(p.sin) && aligned16(p.q_out) && aligned16(p.k_out) &&
                    ((a.qz | a.qh | a.qt | a.kz | a.kh | a.kt | a.cz | a.ct | a.sz | a.st) & 7) == 0;
   if (vec) {
-    const int64_t threads = a.rows * (p.head_dim / 8);
-    hipLaunchKernelGGL(rotary_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, a);
+    const int64_t tokens = rot_tokens(p.head_dim / 16);
+    hipLaunchKernelGGL(rotary_kernel, dim3((unsigned)((a.bt + tokens - 1) / tokens)), dim3(256), 0, stream, a);
   } else {
     const int64_t threads = a.rows * p.head_dim;
     hipLaunchKernelGGL(rotary_kernel_scalar, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, a);
