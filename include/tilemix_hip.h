@@ -171,6 +171,15 @@ typedef struct tilemix_attn_params {
 int tilemix_attn_fwd(const tilemix_attn_params* p, void* stream);
 
 /*
+ * The same for `batch` sequences of `seqlen` tokens each (queries and keys):
+ * sequence z is tokens [z * seqlen, (z + 1) * seqlen), its scale rows start at
+ * z * ceil(seqlen / blk).  No cu array is read (all may be NULL), so the caller
+ * builds none and the workgroups need not wait for them.  max_seqlen_q and
+ * max_seqlen_k must equal seqlen.
+ */
+int tilemix_attn_fwd_uniform(const tilemix_attn_params* p, int32_t seqlen, void* stream);
+
+/*
  * Same computation as tilemix_attn_fwd (same kernel template, a DUMP
  * instantiation), additionally writing, for every computed (row, key) score:
  *   qk_i32[(tok_q) * s_tok + h * s_head + key] = exact int32 Q8.K8 accumulator

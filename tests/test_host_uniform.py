@@ -1,0 +1,47 @@
+"""Argument validation of the uniform-length and several-tensor C entry points (CPU: a
+call that fails validation returns before any HIP call)."""
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+
+from tilemix_amd import _native
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return _native.load_library()
+
+
+def test_uniform_attention_validation(lib):
+    assert lib.tilemix_attn_fwd_uniform(None, 64, None) == 1
+    p = _native.AttnParams()
+    assert lib.tilemix_attn_fwd_uniform(ctypes.byref(p), 0, None) == 1
+    assert b"no tokens" in lib.tilemix_last_error()
+    for f in ("q", "k", "v", "out"):
+        setattr(p, f, ctypes.c_void_p(16))
+    p.max_seqlen_q, p.max_seqlen_k = 64, 65
+    assert lib.tilemix_attn_fwd_uniform(ctypes.byref(p), 64, None) == 1
+    assert b"must equal the uniform length" in lib.tilemix_last_error()
+    p.max_seqlen_k, p.batch = 64, 1 << 26
+    assert lib.tilemix_attn_fwd_uniform(ctypes.byref(p), 64, None) == 1
+    assert b"32-bit token index" in lib.tilemix_last_error()
+    p.batch = 1
+    assert lib.tilemix_attn_fwd(ctypes.byref(p), None) == 1  # without a uniform length: cu arrays needed
+    assert b"cu_seqlens" in lib.tilemix_last_error()
+
+
+def test_several_tensors_validation(lib):
+    q = (_native.QuantParams * 3)()
+    assert lib.tilemix_quant_per_block_int8_many(None, 1, 0, None) == 1
+    for count, uniform in ((0, 0), (4, 0), (1, -1)):
+        assert lib.tilemix_quant_per_block_int8_many(q, count, uniform, None) == 1
+        assert b"1 to 3 tensors" in lib.tilemix_last_error()
+    for s, batch in zip(q, (1, 1, 2)):
+        s.input = s.output = s.scale = 16
+        s.heads, s.head_dim, s.blk_tokens, s.batch = 1, 64, 64, batch
+    assert lib.tilemix_quant_per_block_int8_many(q, 3, 64, None) == 1
+    assert b"share the batch" in lib.tilemix_last_error()
+    assert lib.tilemix_quant_per_block_int8_many(q, 1, 0, None) == 1  # no uniform length: cu_seqlens needed
+    assert b"null tensor pointer" in lib.tilemix_last_error()

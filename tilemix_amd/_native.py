@@ -108,6 +108,7 @@ EXPORTED_SYMBOLS = (
     "tilemix_quant_per_block_int8",
     "tilemix_quant_per_block_int8_many",
     "tilemix_attn_fwd",
+    "tilemix_attn_fwd_uniform",
     "tilemix_attn_fwd_debug",
     "tilemix_rms_norm_f16",
     "tilemix_rotary_f16",
@@ -146,6 +147,8 @@ def load_library(path: os.PathLike | str | None = None) -> ctypes.CDLL:
         lib.tilemix_quant_per_block_int8_many.restype = ctypes.c_int
         lib.tilemix_attn_fwd.argtypes = [ctypes.POINTER(AttnParams), _vp]
         lib.tilemix_attn_fwd.restype = ctypes.c_int
+        lib.tilemix_attn_fwd_uniform.argtypes = [ctypes.POINTER(AttnParams), _i32, _vp]
+        lib.tilemix_attn_fwd_uniform.restype = ctypes.c_int
         lib.tilemix_attn_fwd_debug.argtypes = [ctypes.POINTER(AttnParams), _vp, _vp, _i64, _i64, _vp]
         lib.tilemix_attn_fwd_debug.restype = ctypes.c_int
         lib.tilemix_rms_norm_f16.argtypes = [ctypes.POINTER(RmsNormParams), _vp]
@@ -173,6 +176,31 @@ def load_library(path: os.PathLike | str | None = None) -> ctypes.CDLL:
         if path is None:
             _lib = lib
         return lib
+
+
+_host = None
+
+
+def host():
+    """The native launch path (``tilemix_amd/_host.so``, built from csrc/host.cpp), bound to the
+    library's entry points.  Its functions serve the plain calls and return None for the others."""
+    global _host
+    if _host is not None:
+        return _host
+    lib = load_library()
+    with _lock:
+        if _host is None:
+            try:
+                from . import _host as module
+            except ImportError as e:
+                raise TileMixLibraryError(
+                    f"tilemix_amd/_host.so cannot be loaded ({e}): build it with `python -m tilemix_amd.csrc.build` "
+                    "(or __graft_entry__.build())") from e
+            module.bind(*(ctypes.cast(fn, _vp).value for fn in (
+                lib.tilemix_quant_per_block_int8_many, lib.tilemix_attn_fwd, lib.tilemix_attn_fwd_uniform,
+                lib.tilemix_rms_norm_f16, lib.tilemix_rotary_f16, lib.tilemix_silu_mul_f16)))
+            _host = module
+    return _host
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -50,6 +50,7 @@ ROUTING_MODE_MIXED = _native.ROUTING_MIXED
 ROUTING_MODE_FP16 = _native.ROUTING_FP16
 ROUTING_MODE_INT8 = _native.ROUTING_INT8
 RoutingMode = Literal["auto", "mixed", "fp16", "int8"]
+_MODE_CODES = {"mixed": ROUTING_MODE_MIXED, "fp16": ROUTING_MODE_FP16, "int8": ROUTING_MODE_INT8}
 
 # Tile sizes the gfx950 kernel is instantiated for (block_n > 64 runs as
 # 64-key tiles with the reference's per-block_n softmax step).
@@ -78,6 +79,10 @@ def _quantize_for_caller(items) -> tuple:
     """(codes, scales, scale-row prefix) of each item: one launch, whose kernel writes the scales
     in Q's dtype (fp16, the only one it takes) and the int32 prefixes, and one copy of the row
     counts to the host."""
+    if items[0][0].is_cuda and items[0][1].is_cuda:
+        done = _native.host().quantize(*(arg for item in items for arg in item[:4]))
+        if done is not None:
+            return done
     results, cu_scales = quantize_many(items, half_scales=True)
     out = []
     for (codes, _, scale16), cu_scale, rows in zip(results, cu_scales, scale_rows(items, cu_scales)):
@@ -93,10 +98,9 @@ def _quantize_for_launch(t: torch.Tensor, cu: torch.Tensor, max_seqlen: int, blk
 
 def _routing_mode_code(mode: str) -> int:
     normalized = mode.strip().lower()
-    codes = {"mixed": ROUTING_MODE_MIXED, "fp16": ROUTING_MODE_FP16, "int8": ROUTING_MODE_INT8}
-    if normalized not in codes:
-        raise ValueError(f"routing_mode must be one of {tuple(codes)}, got {mode!r}")
-    return codes[normalized]
+    if normalized not in _MODE_CODES:
+        raise ValueError(f"routing_mode must be one of {tuple(_MODE_CODES)}, got {mode!r}")
+    return _MODE_CODES[normalized]
 
 
 def classify_bitmask_routing(precision_bitmask: torch.Tensor, *, seqlen_q: int, seqlen_k: int,
@@ -476,6 +480,13 @@ def tilemix_attention_with_quant(
         normalized_mode = _classify_cached(
             precision_bitmask, seqlen_q=max_seqlens_q, seqlen_k=max_seqlens_k,
             block_m=block_m, block_n=block_n, block_n_mask=block_n_mask, causal=causal)
+    if bias is None and q.is_cuda and normalized_mode in _MODE_CODES:
+        # The plain call: checks, workspace and launches in one native call (None: not one).
+        out = _native.host().packed(
+            q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlens_q, max_seqlens_k, precision_bitmask, block_m, block_n,
+            block_n_mask, BLKQ, BLKK, causal, sm_scale, _MODE_CODES[normalized_mode], scalar_scales, int8_use_fp16_v)
+        if out is not None:
+            return out, normalized_mode
 
     if normalized_mode == "fp16":
         quantized = _dummy_quantization_metadata(q, k, v, cu_seqlens_q, cu_seqlens_k)

@@ -17,6 +17,7 @@ from typing import Optional
 import torch
 from torch import Tensor
 
+from .. import _native
 from .hip.tilemix import tilemix_attention_with_quant
 
 
@@ -39,6 +40,11 @@ def tilemix_varlen_attention(
 ) -> Tensor:
     """Reference attention/tilemix_varlen.py:17-96 (``candidates`` and
     ``flat_lengths`` are accepted and unused, as there)."""
+    if bias is None and q.is_cuda:
+        # The plain call (token-major tensors or one sequence, see csrc/host.cpp) in one native call.
+        out = _native.host().dense(q, k, v, block_m, block_n, block_n_mask, causal, scale, precision_map_all)
+        if out is not None:
+            return out
     B, Hq, Tq, D = q.shape
     _, Hk, Tk, Dk = k.shape
     _, Hv, Tv, Dv = v.shape

@@ -13,11 +13,23 @@ bool aligned(const void* p, int bytes) { return (reinterpret_cast<uintptr_t>(p) 
 
 }  // namespace
 
-int launch_attn(const tilemix_attn_params& p, int32_t* dump_i32, void* dump_f16, int64_t dump_t,
+int launch_attn(const tilemix_attn_params& p, int uniform_seqlen, int32_t* dump_i32, void* dump_f16, int64_t dump_t,
                 int64_t dump_h, hipStream_t stream) {
-  const char* fn = (dump_i32 || dump_f16) ? "tilemix_attn_fwd_debug" : "tilemix_attn_fwd";
-  if (!p.q || !p.k || !p.v || !p.out || !p.cu_seqlens_q || !p.cu_seqlens_k) {
+  const char* fn = (dump_i32 || dump_f16) ? "tilemix_attn_fwd_debug"
+                   : uniform_seqlen > 0   ? "tilemix_attn_fwd_uniform"
+                                          : "tilemix_attn_fwd";
+  const bool uniform = uniform_seqlen > 0;  // the cu arrays are not read
+  if (!p.q || !p.k || !p.v || !p.out || (!uniform && (!p.cu_seqlens_q || !p.cu_seqlens_k))) {
     set_error("%s: null q/k/v/out/cu_seqlens pointer", fn);
+    return TILEMIX_E_INVALID;
+  }
+  if (uniform && (p.max_seqlen_q != uniform_seqlen || p.max_seqlen_k != uniform_seqlen)) {
+    set_error("%s: max_seqlen_q (%d) and max_seqlen_k (%d) must equal the uniform length %d", fn, p.max_seqlen_q,
+              p.max_seqlen_k, uniform_seqlen);
+    return TILEMIX_E_INVALID;
+  }
+  if (uniform && (int64_t)uniform_seqlen * p.batch > INT32_MAX) {
+    set_error("%s: %d sequences of %d tokens exceed the 32-bit token index", fn, p.batch, uniform_seqlen);
     return TILEMIX_E_INVALID;
   }
   if (p.routing_mode < 0 || p.routing_mode > 2) {
@@ -81,11 +93,11 @@ int launch_attn(const tilemix_attn_params& p, int32_t* dump_i32, void* dump_f16,
                   "block_m 64 without mixed int8-V routing); block_m=%d, BLKQ=%d", fn, p.block_m, p.blkq);
         return TILEMIX_E_INVALID;
       }
-    } else if (!p.q8 || !p.sq || !p.cu_q_scale) {
+    } else if (!p.q8 || !p.sq || (!uniform && !p.cu_q_scale)) {
       set_error("%s: int8 routing needs q8/sq/cu_q_scale (or q_quant_in_kernel)", fn);
       return TILEMIX_E_INVALID;
     }
-    if (!p.k8 || !p.sk || !p.cu_k_scale) {
+    if (!p.k8 || !p.sk || (!uniform && !p.cu_k_scale)) {
       set_error("%s: int8 routing needs k8/sk/cu_k_scale", fn);
       return TILEMIX_E_INVALID;
     }
@@ -101,7 +113,7 @@ int launch_attn(const tilemix_attn_params& p, int32_t* dump_i32, void* dump_f16,
       return TILEMIX_E_INVALID;
     }
     if (int8v) {
-      if (!p.v8 || !p.sv || !p.cu_v_scale) {
+      if (!p.v8 || !p.sv || (!uniform && !p.cu_v_scale)) {
         set_error("%s: int8 V path needs v8/sv/cu_v_scale", fn);
         return TILEMIX_E_INVALID;
       }
@@ -200,6 +212,9 @@ int launch_attn(const tilemix_attn_params& p, int32_t* dump_i32, void* dump_f16,
   a.ng = p.block_n / kBN;
   a.blkq = p.blkq > 0 ? p.blkq : 1;
   a.blkk = p.blkk > 0 ? p.blkk : kBN;
+  a.uni = uniform_seqlen;
+  a.uni_qs = uniform ? (uniform_seqlen - 1) / a.blkq + 1 : 0;
+  a.uni_ks = uniform ? (uniform_seqlen - 1) / a.blkk + 1 : 0;
   // The block_n = 64 kernels take one K/V scale per 64-key tile.
   const bool gen = a.ng > 1 || (need_int8 && a.blkk % kBN != 0);
   a.causal = p.causal ? 1 : 0;

@@ -47,7 +47,28 @@ struct AttnKArgs {
   int per_xcd;
   int pipe;         // the pipelined assembly tile body may serve this launch
   int ilv;          // groups of an XCD interleaved item by item (interleave_groups)
+  int uni;          // > 0: every sequence has this many query and key tokens; no cu array is read
+  int uni_qs, uni_ks;  // uni > 0: Q and K/V scale rows per sequence
 };
+
+// Tokens [start, start + len) of sequence z, and its scale rows [base, end).  With
+// uniform lengths they follow from z: a launch then needs no cu array (nobody
+// builds one) and a workgroup starts without the loads of its bounds.
+struct SeqSpan {
+  int start, len;
+};
+__device__ __forceinline__ SeqSpan seq_span(const int32_t* cu, int uni, int z) {
+  if (uni > 0) return SeqSpan{z * uni, uni};
+  const int start = cu[z];
+  return SeqSpan{start, cu[z + 1] - start};
+}
+struct RowSpan {
+  int base, end;
+};
+__device__ __forceinline__ RowSpan scale_span(const int32_t* cu, int uni, int rows, int z) {
+  if (uni > 0) return RowSpan{z * rows, (z + 1) * rows};
+  return RowSpan{cu[z], cu[z + 1]};
+}
 
 // Work item of workgroup `bid`, or -1.  Items are numbered
 // ((z * hk + kv_head) * m_blocks + mrev) * group + g, so one (sequence, kv head)

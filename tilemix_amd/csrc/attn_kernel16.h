@@ -94,10 +94,9 @@ attn16_kernel(const AttnKArgs a) {
   const int m = a.m_blocks - 1 - mrev;
   const int h = hk * a.group + g;
 
-  const int q_start = a.cu_q[z];
-  const int Lq = a.cu_q[z + 1] - q_start;
-  const int k_start = a.cu_k[z];
-  const int Lk = a.cu_k[z + 1] - k_start;
+  const SeqSpan q_span = seq_span(a.cu_q, a.uni, z), k_span = seq_span(a.cu_k, a.uni, z);
+  const int q_start = q_span.start, Lq = q_span.len;
+  const int k_start = k_span.start, Lk = k_span.len;
   if (m * BM >= Lq) return;
 
   int n_blocks = (Lk + kBN - 1) / kBN;
@@ -141,7 +140,8 @@ attn16_kernel(const AttnKArgs a) {
       if (row_ok && d0 < a.d) raw = *reinterpret_cast<const i32x4*>(qp + d0);
       q8f[s] = raw;
     }
-    const int qb = a.cu_qs[z], qe = a.cu_qs[z + 1];
+    const RowSpan q_rows = scale_span(a.cu_qs, a.uni, a.uni_qs, z);
+    const int qb = q_rows.base, qe = q_rows.end;
     if (qe > qb) {
       const int idx = min(qb + row / a.blkq, qe - 1);
       sq16 = a.sq[(int64_t)idx * a.hq + h];
@@ -157,7 +157,8 @@ attn16_kernel(const AttnKArgs a) {
   // index of each key), fp16, fetched with the tile's copy: one per tile, or
   // (GEN) one per 4-key group of the lane, exact for BLKK divisible by 4.
   auto load_scales = [&](const f16* sc, const int32_t* cus, int n, f16 (&out)[NSG]) {
-    const int base = cus[z], end = cus[z + 1];
+    const RowSpan span = scale_span(cus, a.uni, a.uni_ks, z);
+    const int base = span.base, end = span.end;
 #pragma unroll
     for (int kb = 0; kb < NSG; ++kb) {
       f16 s = (f16)1.0f;

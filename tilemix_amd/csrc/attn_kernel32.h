@@ -129,10 +129,9 @@ attn32_kernel(const AttnKArgs a) {
   const int m = a.m_blocks - 1 - mrev;
   const int h = hk * a.group + g;
 
-  const int q_start = a.cu_q[z];
-  const int Lq = a.cu_q[z + 1] - q_start;
-  const int k_start = a.cu_k[z];
-  const int Lk = a.cu_k[z + 1] - k_start;
+  const SeqSpan q_span = seq_span(a.cu_q, a.uni, z), k_span = seq_span(a.cu_k, a.uni, z);
+  const int q_start = q_span.start, Lq = q_span.len;
+  const int k_start = k_span.start, Lk = k_span.len;
   if (m * BM >= Lq) return;
 
   int n_blocks = (Lk + kBN - 1) / kBN;
@@ -304,15 +303,17 @@ attn32_kernel(const AttnKArgs a) {
   const f16 *skp = nullptr, *sk_last = nullptr, *svp = nullptr, *sv_last = nullptr;
   int ks_base = 0, ks_end = 0, vs_base = 0, vs_end = 0;
   if (MODE != TILEMIX_ROUTING_FP16) {
-    ks_base = a.cu_ks[z];
-    ks_end = a.cu_ks[z + 1];
+    const RowSpan k_rows = scale_span(a.cu_ks, a.uni, a.uni_ks, z);
+    ks_base = k_rows.base;
+    ks_end = k_rows.end;
     has_ks = ks_end > ks_base;
     skp = a.sk + (int64_t)ks_base * a.hk + hk;
     sk_last = a.sk + (int64_t)(ks_end - 1) * a.hk + hk;
   }
   if (INT8V) {
-    vs_base = a.cu_vs[z];
-    vs_end = a.cu_vs[z + 1];
+    const RowSpan v_rows = scale_span(a.cu_vs, a.uni, a.uni_ks, z);
+    vs_base = v_rows.base;
+    vs_end = v_rows.end;
     has_vs = vs_end > vs_base;
     svp = a.sv + (int64_t)vs_base * a.hk + hk;
     sv_last = a.sv + (int64_t)(vs_end - 1) * a.hk + hk;
@@ -541,7 +542,8 @@ attn32_kernel(const AttnKArgs a) {
       if (row_ok && d0 < a.d) raw = *reinterpret_cast<const i32x4*>(qp + d0);
       q8f[s] = raw;
     }
-    const int qb = a.cu_qs[z], qe = a.cu_qs[z + 1];
+    const RowSpan q_rows = scale_span(a.cu_qs, a.uni, a.uni_qs, z);
+    const int qb = q_rows.base, qe = q_rows.end;
     if (qe > qb) {
       const int idx = min(qb + row / a.blkq, qe - 1);
       sq16 = a.sq[(int64_t)idx * a.hq + h];

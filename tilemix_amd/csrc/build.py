@@ -1,9 +1,11 @@
-"""Build libtilemix_hip.so in-tree with hipcc for gfx950.
+"""Build libtilemix_hip.so (hipcc, gfx950) and the host module _host.so in-tree.
 
 Usage: python -m tilemix_amd.csrc.build   (or tilemix_amd.csrc.build.build())
 
 Every .hip file under this directory is compiled to an object in
-tilemix_amd/_build/ (in parallel) and linked into tilemix_amd/libtilemix_hip.so.
+tilemix_amd/_build/ (in parallel) and linked into tilemix_amd/libtilemix_hip.so;
+host.cpp becomes the CPython extension module tilemix_amd/_host.so (the C++
+compiler, against the installed torch).
 """
 from __future__ import annotations
 
@@ -11,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -21,6 +24,7 @@ INCLUDE = REPO / "include"
 BUILD_DIR = PKG / "_build"
 LIB_NAME = "libtilemix_hip.so"
 LIB_PATH = PKG / LIB_NAME
+HOST_PATH = PKG / "_host.so"
 
 ARCH = "gfx950"
 
@@ -66,6 +70,18 @@ def sources() -> list[Path]:
     return sorted(CSRC.glob("*.hip"))
 
 
+def _host_command(out: Path) -> list[str]:
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    includes = [root / "include", root / "include/torch/csrc/api/include", sysconfig.get_paths()["include"],
+                Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "include", INCLUDE]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *(arg for path in includes for arg in ("-isystem", str(path))), str(CSRC / "host.cpp"), "-o", str(out),
+            f"-L{root / 'lib'}", f"-Wl,-rpath,{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> Path:
     """Compile every HIP source for gfx950 and link the shared library."""
     hipcc = _hipcc()
@@ -80,6 +96,8 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
     srcs = sources()
     objs = [BUILD_DIR / (s.stem + ".o") for s in srcs]
     cmds = [[hipcc, *COMMON_FLAGS, "-c", str(s), "-o", str(o)] for s, o in zip(srcs, objs)]
+    host_tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmds.insert(0, _host_command(host_tmp))
     if verbose:
         for c in cmds:
             print(" ".join(c))
@@ -92,6 +110,7 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
         print(" ".join(link))
     _run(link)
     os.replace(tmp, LIB_PATH)
+    os.replace(host_tmp, HOST_PATH)
     return LIB_PATH
 
 

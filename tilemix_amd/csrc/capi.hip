@@ -43,7 +43,15 @@ int tilemix_attn_fwd(const tilemix_attn_params* p, void* stream) {
     tmx::set_error("tilemix_attn_fwd: null params");
     return TILEMIX_E_INVALID;
   }
-  return tmx::launch_attn(*p, nullptr, nullptr, 0, 0, static_cast<hipStream_t>(stream));
+  return tmx::launch_attn(*p, 0, nullptr, nullptr, 0, 0, static_cast<hipStream_t>(stream));
+}
+
+int tilemix_attn_fwd_uniform(const tilemix_attn_params* p, int32_t seqlen, void* stream) {
+  if (p == nullptr || seqlen <= 0) {
+    tmx::set_error("tilemix_attn_fwd_uniform: null params or no tokens (%d)", seqlen);
+    return TILEMIX_E_INVALID;
+  }
+  return tmx::launch_attn(*p, seqlen, nullptr, nullptr, 0, 0, static_cast<hipStream_t>(stream));
 }
 
 int tilemix_attn_fwd_debug(const tilemix_attn_params* p, int32_t* qk_i32, void* qk_f16,
@@ -56,7 +64,7 @@ int tilemix_attn_fwd_debug(const tilemix_attn_params* p, int32_t* qk_i32, void* 
     tmx::set_error("tilemix_attn_fwd_debug: both dump pointers are null");
     return TILEMIX_E_INVALID;
   }
-  return tmx::launch_attn(*p, qk_i32, qk_f16, dump_stride_token, dump_stride_head,
+  return tmx::launch_attn(*p, 0, qk_i32, qk_f16, dump_stride_token, dump_stride_head,
                          static_cast<hipStream_t>(stream));
 }
 

@@ -26,7 +26,7 @@ constexpr float kLog2eF32 = 1.4426950408889634f;
 void set_error(const char* fmt, ...);
 
 int launch_quant(const tilemix_quant_params* ps, int count, int uniform_seqlen, hipStream_t stream);
-int launch_attn(const tilemix_attn_params& p, int32_t* dump_i32, void* dump_f16,
+int launch_attn(const tilemix_attn_params& p, int uniform_seqlen, int32_t* dump_i32, void* dump_f16,
                 int64_t dump_t, int64_t dump_h, hipStream_t stream);
 int launch_rmsnorm(const tilemix_rmsnorm_params& p, hipStream_t stream);
 int launch_rotary(const tilemix_rotary_params& p, hipStream_t stream);

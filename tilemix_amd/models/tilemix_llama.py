@@ -152,6 +152,10 @@ def _require_cuda(what: str, *tensors) -> None:
 def rms_norm(hidden_states, weight, eps: float):
     """HIP RMSNorm over the last dim: weight * fp16(x * rsqrt(mean(x^2) + eps)),
     the mean in fp32 (reference models/tilemix_llama.py:718-797)."""
+    if hidden_states.is_cuda:
+        out = _native.host().rms_norm(hidden_states, weight, eps)
+        if out is not None:
+            return out
     if hidden_states.dtype != torch.float16 or weight.dtype != torch.float16:
         raise ValueError("prefill RMSNorm requires FP16 operands")
     cols = hidden_states.shape[-1]
@@ -195,6 +199,10 @@ def rotary_token_major(q, k, cos, sin):
     returned as ``[b, h, t, d]`` views (reference :808-847): q*cos and
     rotate(q)*sin are each rounded to fp16 and their sum is rounded to fp16.
     One HIP kernel for Q and K."""
+    if q.is_cuda:
+        out = _native.host().rotary(q, k, cos, sin)
+        if out is not None:
+            return out
     b, hq, t, d = q.shape
     hk = k.shape[1]
     if q.dtype != torch.float16 or any(x.dtype != q.dtype for x in (k, cos, sin)):
@@ -224,6 +232,10 @@ def rotary_token_major(q, k, cos, sin):
 
 def silu_mul(gate, up):
     """fp16(silu(gate)) * up in fp32, rounded to fp16 (reference :849-868), one HIP kernel."""
+    if gate.is_cuda:
+        out = _native.host().silu_mul(gate, up)
+        if out is not None:
+            return out
     if gate.dtype != torch.float16 or up.dtype != gate.dtype or gate.shape != up.shape:
         raise ValueError("SiLU requires equally shaped FP16 operands")
     if not gate.is_contiguous() or not up.is_contiguous():
