@@ -491,7 +491,7 @@ PyObject* rotary(PyObject*, PyObject* const* a, Py_ssize_t n) {
   for (int i = 0; i < 4; ++i) {
     x[i] = plain_tensor(a[i], at::kHalf);
     if (x[i] == nullptr || x[i]->dim() != (i < 2 ? 4 : 3) || x[i]->numel() == 0 || x[i]->stride(-1) != 1 ||
-        x[i]->device() != x[0]->device())
+        x[i]->device() != x[0]->device() || x[i]->_fw_grad(0).defined())
       Py_RETURN_NONE;
   }
   const at::Tensor &q = *x[0], &k = *x[1], &cos = *x[2], &sin = *x[3];

@@ -17,7 +17,9 @@ from typing import Optional
 
 import torch
 from torch import Tensor
+from transformers.models.llama.modeling_llama import apply_rotary_pos_emb
 
+from .. import _native
 from ..attention import precision_maps as pm
 
 # Below this many query tokens the module falls back to its parent's attention
@@ -27,6 +29,19 @@ MIN_TILEMIX_SEQLEN = 16
 # Layouts whose percentage-driven map needs no token mask (reference
 # models/tilemix_llama.py:343-359).
 _PERCENTAGE_LAYOUTS = frozenset({"band", "global", "row_rand", "align_sparse", "bigbird", "sptrans"})
+
+
+def apply_rotary(q: Tensor, k: Tensor, cos: Tensor, sin: Tensor):
+    """transformers' ``apply_rotary_pos_emb`` (the same bits) in one HIP kernel for Q and K instead
+    of ten elementwise kernels, where its result carries no graph: fp16 GPU tensors without
+    gradients, outside tracing.  The results are token-major ``[b, t, h, d]`` tensors viewed
+    ``[b, h, t, d]``, the layout the attention call reads without a copy."""
+    if (q.is_cuda and not (torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, cos, sin)))
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()):
+        out = _native.host().rotary(q, k, cos, sin)
+        if out is not None:
+            return out
+    return apply_rotary_pos_emb(q, k, cos, sin)
 
 
 @dataclass(frozen=True)

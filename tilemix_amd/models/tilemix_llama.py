@@ -20,12 +20,12 @@ from typing import Optional, Tuple
 import torch
 from torch import Tensor, nn
 from transformers.cache_utils import Cache, DynamicLayer
-from transformers.models.llama.modeling_llama import LlamaAttention, apply_rotary_pos_emb
+from transformers.models.llama.modeling_llama import LlamaAttention
 
 from .. import _native
 from ..attention.tilemix_varlen import tilemix_varlen_attention
-from ._common import (MIN_TILEMIX_SEQLEN, BucketConfig, TileMixRoutingMixin, pick_block_n_for_64,  # noqa: F401
-                      pick_mask_block_n)
+from ._common import (MIN_TILEMIX_SEQLEN, BucketConfig, TileMixRoutingMixin, apply_rotary,  # noqa: F401
+                      pick_block_n_for_64, pick_mask_block_n)
 
 __all__ = ["TileMixLlamaAttention", "inject_tilemix_into_llama", "configure_tilemix_attention_pattern", "rms_norm",
            "PrefillCache", "prepare_llama_prefill", "prepare_llama_norms", "rotary_token_major", "silu_mul",
@@ -36,7 +36,7 @@ __all__ = ["TileMixLlamaAttention", "inject_tilemix_into_llama", "configure_tile
 class TileMixLlamaAttention(TileMixRoutingMixin, LlamaAttention):
     """Reference models/tilemix_llama.py:52-646."""
 
-    apply_rotary = staticmethod(apply_rotary_pos_emb)
+    apply_rotary = staticmethod(apply_rotary)
 
     def __init__(self, config, layer_idx: int):
         LlamaAttention.__init__(self, config, layer_idx=layer_idx)

@@ -13,10 +13,10 @@ from typing import Optional, Tuple
 
 import torch
 from torch import Tensor
-from transformers.models.qwen2.modeling_qwen2 import Qwen2Attention, apply_rotary_pos_emb
+from transformers.models.qwen2.modeling_qwen2 import Qwen2Attention
 
 from ..attention.tilemix_varlen import tilemix_varlen_attention
-from ._common import MIN_TILEMIX_SEQLEN, TileMixRoutingMixin
+from ._common import MIN_TILEMIX_SEQLEN, TileMixRoutingMixin, apply_rotary
 from .tilemix_llama import _swap_attention
 
 __all__ = ["TileMixqwenAttention", "inject_tilemix_into_qwen", "configure_tilemix_attention_pattern",
@@ -86,14 +86,13 @@ class TileMixqwenAttention(TileMixRoutingMixin, Qwen2Attention):
         else:
             cos, sin = self.rotary_emb(q, kwargs.get("position_ids"))
         cos, sin = cos.to(device), sin.to(device)
-        q, k = apply_rotary_pos_emb(q, k, cos, sin)
+        q, k = apply_rotary(q, k, cos, sin)
         if past_key_values is not None:
             k, v = past_key_values.update(k, v, self.layer_idx,
                                           cache_kwargs={"sin": sin, "cos": cos, "cache_position": cache_position})
         assert q.shape[1] == self.nh, f"Q heads {q.shape[1]} != nh {self.nh}"
         assert k.shape[1] == self.nkv, f"K heads {k.shape[1]} != nkv {self.nkv}"
         assert v.shape[1] == self.nkv, f"V heads {v.shape[1]} != nkv {self.nkv}"
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
 
         out = tilemix_varlen_attention(q, k, v, cfg.block_m, cfg.block_n, block_n_mask=block_n_mask, causal=True,
                                        scale=head_dim ** -0.5, precision_map_all=clean,
