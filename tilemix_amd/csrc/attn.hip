@@ -220,21 +220,20 @@ int launch_attn(const tilemix_attn_params& p, int uniform_seqlen, int32_t* dump_
   a.causal = p.causal ? 1 : 0;
   a.q_fused = (need_int8 && p.q_quant_in_kernel) ? 1 : 0;
   const bool dump = dump_i32 != nullptr || dump_f16 != nullptr;
-  a.total_items = (int)total;
   // The pipelined assembly tile body (head_dim 128, 128-row workgroups, fp16 V,
   // no bias, block_n 64); TILEMIX_HIP_PIPE=0 selects the C++ tile body.
   {
     const char* env = getenv("TILEMIX_HIP_PIPE");
     a.pipe = (env != nullptr && env[0] == '0') ? 0 : 1;
   }
-  a.per_xcd = (int)work_items_per_xcd((int64_t)p.heads_k * p.batch, (int64_t)m_blocks * a.group);
   // Groups interleaved per XCD (the work order only: outputs do not depend on
   // it); TILEMIX_HIP_INTERLEAVE=1..4 overrides the choice.
-  a.ilv = interleave_groups(p.max_seqlen_k, p.head_dim);
+  int ilv = interleave_groups(p.max_seqlen_k, p.head_dim);
   {
     const char* env = getenv("TILEMIX_HIP_INTERLEAVE");
-    if (env != nullptr && env[0] >= '1' && env[0] <= '4' && env[1] == '\0') a.ilv = env[0] - '0';
+    if (env != nullptr && env[0] >= '1' && env[0] <= '4' && env[1] == '\0') ilv = env[0] - '0';
   }
+  a.work = make_work_map((int)total, m_blocks * a.group, ilv, a.group, p.heads_k);
 
   const int dp = p.head_dim <= 64 ? 64 : 128;
   dispatch_attn(a, kind, dp, p.routing_mode, int8v, dump, p.bias != nullptr, gen, stream);

@@ -10,6 +10,95 @@ namespace tmx {
 
 constexpr int kBN = 64;  // keys per compute tile (block_n)
 
+// n / d for 0 <= n < 2^31 by a multiplication: with 2^shift the smallest power of
+// two >= d, q = (n + hi32(n * mul)) >> shift (three scalar instructions where a
+// division by a kernel argument takes about thirty, in series).
+struct FastDiv {
+  uint32_t mul;
+  int shift, d;
+};
+inline FastDiv make_fast_div(int d) {
+  int shift = 0;
+  while (((int64_t)1 << shift) < d) ++shift;
+  return FastDiv{(uint32_t)(((((uint64_t)1 << shift) - (uint64_t)d) << 32) / (uint64_t)d + 1), shift, d};
+}
+__host__ __device__ __forceinline__ int fast_div(int n, const FastDiv& f) {
+  return (int)(((uint32_t)(((uint64_t)(uint32_t)n * f.mul) >> 32) + (uint32_t)n) >> f.shift);
+}
+
+// Work item of workgroup `bid`, or none.  Items are numbered
+// ((z * hk + kv_head) * m_blocks + mrev) * group + g, so one (sequence, kv head)
+// "group" is ipg = m_blocks * group consecutive items, its query blocks
+// longest first.  Workgroups reach the 8 XCDs round-robin (bid & 7); the j-th
+// workgroup of XCD x takes
+//   * while whole rounds of 8 groups remain: from XCD x's groups x, x + 8,
+//     x + 16, ... -- a group stays on one XCD (its L2 serves every re-read of
+//     the group's K/V tiles) and groups are dealt round-robin, so every XCD
+//     gets the same mix of long and short sequences.  The XCD's groups run ilv
+//     at a time, interleaved item by item (chunk c = j / (ilv ipg) holds groups
+//     c ilv .. c ilv + kc - 1, kc = min(ilv, groups left); position w = j mod
+//     (ilv ipg) takes item w / kc of group c ilv + w mod kc): the last items
+//     dispatched are then the short query blocks of ilv groups instead of
+//     every block of the last group, which shortens the launch's tail, as
+//     long as ilv groups' K/V stay in the XCD's L2 (interleave_groups);
+//   * for the last G % 8 groups: their items dealt over all 8 XCDs (position
+//     8 j' + x), which also covers a launch with fewer than 8 groups.
+// per_xcd (the grid is 8 * per_xcd) = (G / 8) * ipg + ceil((G % 8) * ipg / 8).
+__host__ __device__ inline int64_t work_items_per_xcd(int64_t groups, int64_t ipg) {
+  return (groups / 8) * ipg + ((groups % 8) * ipg + 7) / 8;
+}
+// The mapping's constants, computed once per launch on the host.
+struct WorkMap {
+  int ipg, ilv;
+  int gpx;      // whole-round groups per XCD
+  int tail;     // groups after the whole rounds
+  int full_j;  // workgroups per XCD in whole rounds
+  int per_xcd;  // workgroups per XCD
+  FastDiv by_chunk, by_ilv, by_last, by_ipg;  // ilv ipg, ilv, kc of the last chunk, ipg
+  FastDiv by_group, by_hk;                          // query heads per KV head, KV heads
+};
+inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int hk) {
+  WorkMap w;
+  w.ipg = ipg;
+  w.ilv = ilv;
+  w.gpx = total_items / ipg / 8;
+  w.tail = total_items / ipg % 8;
+  w.full_j = w.gpx * ipg;
+  w.per_xcd = (int)work_items_per_xcd(total_items / ipg, ipg);
+  const int64_t chunk = (int64_t)ilv * ipg;
+  w.by_chunk = make_fast_div(chunk < INT32_MAX ? (int)chunk : INT32_MAX);
+  w.by_ilv = make_fast_div(ilv);
+  w.by_last = make_fast_div(w.gpx % ilv != 0 ? w.gpx % ilv : ilv);
+  w.by_ipg = make_fast_div(ipg);
+  w.by_group = make_fast_div(group);
+  w.by_hk = make_fast_div(hk);
+  return w;
+}
+// The group of workgroup `bid` and its item in the group; false: no item.
+__host__ __device__ __forceinline__ bool work_position(const WorkMap& w, int bid, int& grp, int& item) {
+  const int x = bid & 7, j = bid >> 3;
+  if (j < w.full_j) {
+    const int c = fast_div(j, w.by_chunk);
+    const int p = j - c * w.by_chunk.d;
+    const bool last = w.gpx - c * w.ilv < w.ilv;
+    const FastDiv by_kc = last ? w.by_last : w.by_ilv;
+    item = fast_div(p, by_kc);
+    grp = x + 8 * (c * w.ilv + p - item * by_kc.d);
+    return true;
+  }
+  const int n = 8 * (j - w.full_j) + x;
+  grp = fast_div(n, w.by_ipg);
+  item = n - grp * w.ipg;
+  grp += 8 * w.gpx;
+  return n < w.tail * w.ipg;
+}
+// The same as an item number, or -1.
+inline int work_item(int bid, int total_items, int ipg, int ilv) {
+  const WorkMap w = make_work_map(total_items, ipg, ilv, 1, 1);
+  int grp, item;
+  return work_position(w, bid, grp, item) ? grp * ipg + item : -1;
+}
+
 struct AttnKArgs {
   const f16* q;
   const f16* k;
@@ -43,10 +132,8 @@ struct AttnKArgs {
   int blkq, blkk;
   int causal;
   int q_fused;      // Q quantised in the attention kernel (128-row workgroups, BLKQ == 128)
-  int total_items;  // (sequence, query head, query block) work items
-  int per_xcd;
+  WorkMap work;     // workgroup -> (sequence, query head, query block)
   int pipe;         // the pipelined assembly tile body may serve this launch
-  int ilv;          // groups of an XCD interleaved item by item (interleave_groups)
   int uni;          // > 0: every sequence has this many query and key tokens; no cu array is read
   int uni_qs, uni_ks;  // uni > 0: Q and K/V scale rows per sequence
 };
@@ -70,42 +157,6 @@ __device__ __forceinline__ RowSpan scale_span(const int32_t* cu, int uni, int ro
   return RowSpan{cu[z], cu[z + 1]};
 }
 
-// Work item of workgroup `bid`, or -1.  Items are numbered
-// ((z * hk + kv_head) * m_blocks + mrev) * group + g, so one (sequence, kv head)
-// "group" is ipg = m_blocks * group consecutive items, its query blocks
-// longest first.  Workgroups reach the 8 XCDs round-robin (bid & 7); the j-th
-// workgroup of XCD x takes
-//   * while whole rounds of 8 groups remain: from XCD x's groups x, x + 8,
-//     x + 16, ... -- a group stays on one XCD (its L2 serves every re-read of
-//     the group's K/V tiles) and groups are dealt round-robin, so every XCD
-//     gets the same mix of long and short sequences.  The XCD's groups run ilv
-//     at a time, interleaved item by item (chunk c = j / (ilv ipg) holds groups
-//     c ilv .. c ilv + kc - 1, kc = min(ilv, groups left); position w = j mod
-//     (ilv ipg) takes item w / kc of group c ilv + w mod kc): the last items
-//     dispatched are then the short query blocks of ilv groups instead of
-//     every block of the last group, which shortens the launch's tail, as
-//     long as ilv groups' K/V stay in the XCD's L2 (interleave_groups);
-//   * for the last G % 8 groups: their items dealt over all 8 XCDs (item
-//     8 j' + x), which also covers a launch with fewer than 8 groups.
-// per_xcd (the grid is 8 * per_xcd) = (G / 8) * ipg + ceil((G % 8) * ipg / 8).
-__host__ __device__ inline int64_t work_items_per_xcd(int64_t groups, int64_t ipg) {
-  return (groups / 8) * ipg + ((groups % 8) * ipg + 7) / 8;
-}
-__host__ __device__ __forceinline__ int work_item(int bid, int total_items, int ipg, int ilv) {
-  const int x = bid & 7, j = bid >> 3;
-  const int groups = total_items / ipg;
-  const int gpx = groups / 8;            // whole-round groups per XCD
-  const int full_j = gpx * ipg;          // workgroups per XCD in whole rounds
-  if (j < full_j) {
-    const int c = j / (ilv * ipg);
-    const int kc = min(ilv, gpx - c * ilv);
-    const int w = j - c * ilv * ipg;
-    return (x + 8 * (c * ilv + w % kc)) * ipg + w / kc;
-  }
-  const int item = gpx * 8 * ipg + 8 * (j - full_j) + x;
-  return item < total_items ? item : -1;
-}
-
 // Groups interleaved per XCD (work_item): as many as keep their K/V tiles
 // (fp16 K and V, int8 K: 5 bytes per key and head-dim column) within ~5.5 MB,
 // a little over one XCD's 4 MB L2, at most 4.  Measured on cfg2-like
@@ -119,6 +170,7 @@ __host__ __device__ inline int interleave_groups(int64_t max_seqlen_k, int head_
 }
 
 typedef __attribute__((address_space(3))) void lds_void;
+typedef short s16x2 __attribute__((ext_vector_type(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 
@@ -216,6 +268,57 @@ __device__ __forceinline__ float div_by_recip(float x, float s, float r) {
   const float q0 = x * r;
   const float rem = __builtin_fmaf(-q0, s, x);
   return __builtin_fmaf(rem, r, q0);
+}
+
+// The int8 codes of fp16 values x and block scale s, r = RN(1/s) (0 for an all-zero
+// block, whose codes come out as 0): trunc(x / s + (x < 0 ? -0.5 : 0.5)), the
+// quotient as in div_by_recip with the fp16 operand converted inside the FMAs
+// (one rounding each, as on the converted value).  The sign of the half is x's:
+// a quotient of -0 truncates to 0 either way.
+__device__ __forceinline__ float rem_lo(uint32_t h2, float q0, float s) {
+  float r;
+  asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel_hi:[0,0,1]" : "=v"(r) : "v"(q0), "v"(s), "v"(h2));
+  return r;
+}
+__device__ __forceinline__ float rem_hi(uint32_t h2, float q0, float s) {
+  float r;
+  asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r) : "v"(q0), "v"(s), "v"(h2));
+  return r;
+}
+__device__ __forceinline__ float add_lo(float t, uint32_t h2) {
+  float r;
+  asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[0,0,1]" : "=v"(r) : "v"(t), "v"(h2));
+  return r;
+}
+__device__ __forceinline__ float add_hi(float t, uint32_t h2) {
+  float r;
+  asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r) : "v"(t), "v"(h2));
+  return r;
+}
+// The rounded-away values of the pair x (truncate them to get the codes).
+__device__ __forceinline__ void quotient_pair(uint32_t x, float s, float r, float* v) {
+  const uint32_t half = (x & 0x80008000u) | 0x38003800u;  // +-0.5
+  const float a = mul_lo(x, r), b = mul_hi(x, r);
+  v[0] = add_lo(__builtin_fmaf(rem_lo(x, a, s), r, a), half);
+  v[1] = add_hi(__builtin_fmaf(rem_hi(x, b, s), r, b), half);
+}
+// trunc of eight values as the bytes of two words: the conversions write their
+// byte of the word themselves (a byte write is read by the next write of the same
+// word two instructions later, and by nothing before the final s_nop).
+__device__ __forceinline__ uint2 trunc_bytes(const float* v) {
+  uint2 w;
+  asm("v_cvt_i32_f32_sdwa %0, %2 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD\n\t"
+      "v_cvt_i32_f32_sdwa %1, %6 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD\n\t"
+      "v_cvt_i32_f32_sdwa %0, %3 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD\n\t"
+      "v_cvt_i32_f32_sdwa %1, %7 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD\n\t"
+      "v_cvt_i32_f32_sdwa %0, %4 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:DWORD\n\t"
+      "v_cvt_i32_f32_sdwa %1, %8 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:DWORD\n\t"
+      "v_cvt_i32_f32_sdwa %0, %5 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:DWORD\n\t"
+      "v_cvt_i32_f32_sdwa %1, %9 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:DWORD\n\t"
+      "s_nop 0"
+      : "=&v"(w.x), "=&v"(w.y)
+      : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]));
+  return w;
 }
 
 // Lane pairs (l, l^16) and (l, l^32): returns {value of the lower lane, value

@@ -81,16 +81,10 @@ attn16_kernel(const AttnKArgs a) {
   const int lg = lane >> 4;  // key group
 
   // ---- work item ---------------------------------------------------------
-  const int bid = blockIdx.x;
-  const int lam = work_item(bid, a.total_items, a.m_blocks * a.group, a.ilv);
-  if (lam < 0) return;
-  int t = lam;
-  const int g = t % a.group;
-  t /= a.group;
-  const int mrev = t % a.m_blocks;
-  t /= a.m_blocks;
-  const int hk = t % a.hk;
-  const int z = t / a.hk;
+  int grp, item;
+  if (!work_position(a.work, blockIdx.x, grp, item)) return;
+  const int mrev = fast_div(item, a.work.by_group), g = item - mrev * a.group;
+  const int z = fast_div(grp, a.work.by_hk), hk = grp - z * a.hk;
   const int m = a.m_blocks - 1 - mrev;
   const int h = hk * a.group + g;
 

@@ -115,17 +115,13 @@ attn32_kernel(const AttnKArgs a) {
   const int l32 = lane & 31;
   const int hi = lane >> 5;
 
+  const float qk_scale = a.qk_scale;
+
   // ---- work item ---------------------------------------------------------
-  const int bid = blockIdx.x;
-  const int lam = work_item(bid, a.total_items, a.m_blocks * a.group, a.ilv);
-  if (lam < 0) return;
-  int t = lam;
-  const int g = t % a.group;
-  t /= a.group;
-  const int mrev = t % a.m_blocks;
-  t /= a.m_blocks;
-  const int hk = t % a.hk;
-  const int z = t / a.hk;
+  int grp, item;
+  if (!work_position(a.work, blockIdx.x, grp, item)) return;
+  const int mrev = fast_div(item, a.work.by_group), g = item - mrev * a.group;
+  const int z = fast_div(grp, a.work.by_hk), hk = grp - z * a.hk;
   const int m = a.m_blocks - 1 - mrev;
   const int h = hk * a.group + g;
 
@@ -463,7 +459,7 @@ attn32_kernel(const AttnKArgs a) {
       const u32x4 w = __builtin_bit_cast(u32x4, qraw[s]);
       u32x4 o;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = pack_h2(mul_lo(w[r], a.qk_scale), mul_hi(w[r], a.qk_scale));
+      for (int r = 0; r < 4; ++r) o[r] = pack_h2(mul_lo(w[r], qk_scale), mul_hi(w[r], qk_scale));
       qf[s] = __builtin_bit_cast(f16x8, o);
     }
   }
@@ -500,7 +496,7 @@ attn32_kernel(const AttnKArgs a) {
 #pragma unroll
     for (int w = 1; w < NW; ++w) am = fmaxf(am, q_red[w]);
     const float qs = am / 127.0f;  // IEEE division
-    const float qr = 1.0f / qs;    // IEEE reciprocal (inf when qs == 0: codes are 0 then)
+    const float qr = qs == 0.0f ? 0.0f : 1.0f / qs;  // IEEE reciprocal (an all-zero block: codes 0)
     sq16 = (f16)qs;
     // fp16 layout -> int8 layout: lanes l and l+32 exchange one half of each
     // pair of fp16 k-steps (2 s, 2 s + 1), so each lane then holds
@@ -515,23 +511,14 @@ attn32_kernel(const AttnKArgs a) {
         x[r] = sw[0];
         y[r] = sw[1];
       }
-      const f16x8 xv = __builtin_bit_cast(f16x8, x), yv = __builtin_bit_cast(f16x8, y);
-      uint32_t w[4] = {0u, 0u, 0u, 0u};
-      const u32x4 xw = __builtin_bit_cast(u32x4, xv), yw = __builtin_bit_cast(u32x4, yv);
+      float v[16];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        // div_by_recip with q0 = RN(x r) straight from the fp16 operand
-        const uint32_t h2 = e < 8 ? xw[(e & 7) >> 1] : yw[(e & 7) >> 1];
-        const float x = (float)(e < 8 ? xv[e] : yv[e - 8]);
-        const float q0 = (e & 1) ? mul_hi(h2, qr) : mul_lo(h2, qr);
-        float t = __builtin_fmaf(__builtin_fmaf(-q0, qs, x), qr, q0);
-        // t + (t >= 0 ? 0.5 : -0.5); they differ only at t = -0, where both
-        // truncate to code 0
-        t += __builtin_copysignf(0.5f, t);
-        const int code = (qs == 0.0f) ? 0 : (int)t;
-        w[e >> 2] |= (uint32_t)(code & 0xff) << (8 * (e & 3));
+      for (int r = 0; r < 4; ++r) {
+        quotient_pair(x[r], qs, qr, v + 2 * r);
+        quotient_pair(y[r], qs, qr, v + 8 + 2 * r);
       }
-      q8f[s] = (i32x4){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+      const uint2 lo = trunc_bytes(v), hi8 = trunc_bytes(v + 8);
+      q8f[s] = (i32x4){(int)lo.x, (int)lo.y, (int)hi8.x, (int)hi8.y};
     }
   } else if (MODE != TILEMIX_ROUTING_FP16) {
     const int8_t* qp = a.q8 + (int64_t)(q_start + row) * a.sq8_t + (int64_t)h * a.sq8_h;
@@ -649,7 +636,7 @@ attn32_kernel(const AttnKArgs a) {
 #pragma unroll
       for (int g = 0; g < NSG; ++g) {
         const f16 sqk = sq16 * skc[g];
-        ss[g] = fp32_round((float)(f16)fp32_round((float)sqk * a.qk_scale));
+        ss[g] = fp32_round((float)(f16)fp32_round((float)sqk * qk_scale));
         negms[g] = -kMagic * ss[g];
       }
       int kbase8 = l32 * ROW8 + ((16 * hi) ^ (16 * swz_k<ROW8>(l32)));
@@ -706,7 +693,25 @@ attn32_kernel(const AttnKArgs a) {
   // ---- mask + optional bias ------------------------------------------------
   auto tile_mask = [&](int key0, uint32_t (&s16)[2][8]) {
     const bool need_mask = (key0 + kBN > Lk) || (a.causal && key0 + kBN - 1 > row0w + diag);
-    if (need_mask || BIAS) {
+    if (!BIAS && need_mask) {
+      // Key c of the lane's 64-key pattern (less its 4 hi) is valid iff c <= rel.
+      // Both keys of a packed pair at once: the sign of rel - c is the invalid
+      // half's mask, which selects -inf (three instructions a pair; a compare and
+      // a select per score wait on each other's condition registers).
+      const int lim = a.causal ? min(Lk - 1, row + diag) : Lk - 1;  // last valid key
+      const short rel = (short)min(max(lim - key0 - 4 * hi, -1), kBN);
+      const s16x2 rel2 = {rel, rel};
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const short c = (short)(kb * 32 + 8 * (j >> 1) + 2 * (j & 1));
+          const s16x2 left = rel2 - (s16x2){c, (short)(c + 1)};
+          const uint32_t bad = __builtin_bit_cast(uint32_t, left >> 15);
+          s16[kb][j] = (s16[kb][j] & ~bad) | (bad & 0xfc00fc00u);
+        }
+    }
+    if (BIAS) {
       const int lim = a.causal ? min(Lk - 1, row + diag) : Lk - 1;  // last valid key
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
@@ -719,7 +724,7 @@ attn32_kernel(const AttnKArgs a) {
             const int key = key0 + kb * 32 + 8 * (rr >> 2) + 4 * hi + (rr & 3);
             if (key > lim) {
               pr[e] = (f16)(-INFINITY);
-            } else if (BIAS && row_ok) {
+            } else if (row_ok) {
               // Reference :264-272: qk(fp16) += fp16(b * LOG2E) with LOG2E taken
               // as an fp16 constant against the fp16 bias (weak scalar typing);
               // the bias row pointer carries no batch offset (quirk kept).
@@ -908,7 +913,7 @@ attn32_kernel(const AttnKArgs a) {
       c.dk8 = dma_k8;
       c.dv16 = dma_v16;
       c.sq16 = __builtin_bit_cast(uint16_t, sq16);
-      c.qks = a.qk_scale;
+      c.qks = qk_scale;
       c.magic2 = 0x4B4000004B400000ull;
       if constexpr (MODE != TILEMIX_ROUTING_FP16) {
         // K scales through a raw buffer over the whole array (every lookup is
@@ -1033,7 +1038,12 @@ attn32_kernel(const AttnKArgs a) {
     l_i = sw.x + sw.y;
   }
   if (row_ok) {
-    f16* op = a.out + (int64_t)(q_start + row) * a.so_t + (int64_t)h * a.so_h;
+    // The epilogue's arguments are read again here: kept from the start, they cost
+    // the tile loop scalar registers, and the register-starved instantiations
+    // (int8 V, mixed) spilled 12 to 96 of them.
+    const AttnKArgs* late = (const AttnKArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(late));
+    f16* op = late->out + (int64_t)(q_start + row) * late->so_t + (int64_t)h * late->so_h;
     // acc / l from one IEEE reciprocal per row and Markstein's correction
     // step per element (3 instructions instead of a full division each); the
     // quotient is the correctly rounded one (checked against exact rational
@@ -1041,18 +1051,28 @@ attn32_kernel(const AttnKArgs a) {
     // barrier keeps it an fp32 value: folded into one mixed-precision FMA
     // that rounds straight to fp16, it would differ on double-rounding ties.
     const float rl = 1.0f / l_i;
+    auto quad = [&](int db, int rq) {
+      f16x4 o;
 #pragma unroll
-    for (int db = 0; db < NDB; ++db)
+      for (int e = 0; e < 4; ++e) o[e] = (f16)fp32_round(div_by_recip(acc[db][4 * rq + e], l_i, rl));
+      return o;
+    };
+    // The stores share one address with constant offsets; a row narrower than DP
+    // ends at a multiple of 16 columns, the same for every lane (scalar branches).
+    f16* oh = op + 4 * hi;
+    const int d = late->d;
+    if (d == DP) {
 #pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        const int d0 = db * 32 + 8 * rq + 4 * hi;
-        if (d0 < a.d) {
-          f16x4 o;
+      for (int db = 0; db < NDB; ++db)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = (f16)fp32_round(div_by_recip(acc[db][4 * rq + e], l_i, rl));
-          *reinterpret_cast<f16x4*>(op + d0) = o;
-        }
-      }
+        for (int rq = 0; rq < 4; ++rq) *reinterpret_cast<f16x4*>(oh + db * 32 + 8 * rq) = quad(db, rq);
+    } else {
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq)
+          if (db * 32 + 16 * (rq >> 1) < d) *reinterpret_cast<f16x4*>(oh + db * 32 + 8 * rq) = quad(db, rq);
+    }
   }
 }
 

@@ -11,7 +11,7 @@ template <bool DUMP, bool BIAS, bool GEN>
 struct AttnLauncher {
   template <int DP, int MODE, bool INT8V>
   static void one(const AttnKArgs& a, int kind, hipStream_t stream) {
-    const dim3 grid(8 * a.per_xcd), block(256);
+    const dim3 grid(8 * a.work.per_xcd), block(256);
     if constexpr (MODE == TILEMIX_ROUTING_MIXED && INT8V) {
       if (kind == kAttn16) {
         hipLaunchKernelGGL((attn16_kernel<4, DP, MODE, INT8V, DUMP, BIAS, GEN>), grid, block, 0, stream, a);

@@ -17,8 +17,8 @@
 // What bounds it: HBM (2 bytes read, 1 written per element), closely followed by
 // VALU issue, so the arithmetic is kept small: a thread's rows differ by a
 // uniform stride (no division per 16-byte chunk), the block maximum is taken on
-// packed 16-bit magnitudes, and a code costs ~7 instructions (mixed-precision
-// FMAs straight from the fp16 operand, byte permutes).  Heads are the fastest
+// packed 16-bit magnitudes, and a code costs 5.5 instructions (mixed-precision
+// FMAs straight from the fp16 operand, conversions that write their byte).  Heads are the fastest
 // block index, so the workgroups in flight read neighbouring 256-byte rows.
 // Against a kernel with a 32-bit division per chunk, fp32 maxima reduced through
 // LDS, the scale-row prefix (and its barrier) before the loads, and ~12 instructions
@@ -63,18 +63,6 @@ __device__ __forceinline__ uint32_t pk_max_u16(uint32_t x, uint32_t y) {
   return r;
 }
 
-// fp32(h) - q0 * s with one rounding, for the low / high fp16 half of h2.
-__device__ __forceinline__ float rem_lo(uint32_t h2, float q0, float s) {
-  float r;
-  asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel_hi:[0,0,1]" : "=v"(r) : "v"(q0), "v"(s), "v"(h2));
-  return r;
-}
-__device__ __forceinline__ float rem_hi(uint32_t h2, float q0, float s) {
-  float r;
-  asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r) : "v"(q0), "v"(s), "v"(h2));
-  return r;
-}
-
 // Maximum over the wave (every lane gets it): lanes l ^ 32 and l ^ 16 by
 // permlane swaps, the rest of a 16-lane row by DPP moves.
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
@@ -93,12 +81,6 @@ __device__ __forceinline__ int wave_sum_i(int v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
-}
-
-// Four codes to bytes of one word.
-__device__ __forceinline__ uint32_t pack4(const int* c) {
-  return __builtin_amdgcn_perm((uint32_t)c[1], (uint32_t)c[0], 0x0c0c0400u) |
-         __builtin_amdgcn_perm((uint32_t)c[3], (uint32_t)c[2], 0x04000c0cu);
 }
 
 __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(const QuantKArgs args) {
@@ -154,30 +136,20 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
   // directly.
   const bool unit_scale = sm == 1.0f;
   auto encode = [&](const u32x4& x, float s, float rs, int8_t* dst) {
-    int c[8];
+    float v[8];
     if (unit_scale) {
       // rs is 0 for an all-zero block, whose codes then come out as 0.
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t h2 = x[e >> 1];
-        const float q0 = (e & 1) ? mul_hi(h2, rs) : mul_lo(h2, rs);
-        const float rem = (e & 1) ? rem_hi(h2, q0, s) : rem_lo(h2, q0, s);
-        float v = __builtin_fmaf(rem, rs, q0);
-        // v + (v >= 0 ? 0.5 : -0.5); they differ only at v = -0, where both
-        // truncate to code 0.
-        v += __builtin_copysignf(0.5f, v);
-        c[e] = (int)v;
-      }
+      for (int e = 0; e < 4; ++e) quotient_pair(x[e], s, rs, v + 2 * e);
     } else {
       const f16x8 xv = __builtin_bit_cast(f16x8, x);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        float v = ((float)xv[e] * sm) / s;
-        v += (v >= 0.0f) ? 0.5f : -0.5f;
-        c[e] = (s == 0.0f) ? 0 : (int)v;
+        const float t = ((float)xv[e] * sm) / s;
+        v[e] = s == 0.0f ? 0.0f : t + ((t >= 0.0f) ? 0.5f : -0.5f);
       }
     }
-    *reinterpret_cast<uint2*>(dst) = make_uint2(pack4(c), pack4(c + 4));
+    *reinterpret_cast<uint2*>(dst) = trunc_bytes(v);
   };
   // max|x * sm| over the block from the lane's largest magnitude (packed 16-bit
   // patterns without their signs order like the values; RN(x * sm) is monotonic
