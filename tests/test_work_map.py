@@ -1,0 +1,61 @@
+"""The order in which workgroups take work items (attn_common.h: spread_workgroup and
+work_position), compiled for the host and checked on the CPU: every item once, a whole
+round's group on one XCD, each shader engine's share of every group, launches of fewer
+than 8 groups starting with the longest query blocks of each; and fast_div."""
+from __future__ import annotations
+
+import shutil
+import subprocess
+from collections import Counter
+from pathlib import Path
+
+import pytest
+
+REPO = Path(__file__).resolve().parent.parent
+
+
+@pytest.fixture(scope="module")
+def dump_bin(tmp_path_factory):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).exists():
+        pytest.skip("hipcc not available")
+    out = tmp_path_factory.mktemp("wm") / "work_map_dump"
+    subprocess.run([hipcc, "--offload-arch=gfx950", "-O1", "-std=c++17", f"-I{REPO / 'include'}",
+                    f"-I{REPO / 'tilemix_amd' / 'csrc'}", str(REPO / "tests" / "native" / "work_map_dump.cpp"),
+                    "-o", str(out)], check=True, capture_output=True)
+    return out
+
+
+def _run(dump_bin, *args):
+    return subprocess.run([str(dump_bin), *map(str, args)], check=True, capture_output=True, text=True).stdout
+
+
+def test_fast_div(dump_bin):
+    assert int(_run(dump_bin, "--div")) == 0
+
+
+@pytest.mark.parametrize("ilv", [1, 2, 3, 4])
+@pytest.mark.parametrize("groups,m_blocks,group", [(64, 32, 3), (64, 15, 4), (4, 13, 7), (13, 5, 2), (9, 7, 1),
+                                                   (7, 1, 1), (1, 1, 1), (24, 3, 5), (8, 2, 8), (3, 256, 7)])
+def test_launch_order(dump_bin, groups, m_blocks, group, ilv):
+    rows = [tuple(map(int, ln.split())) for ln in _run(dump_bin, groups, m_blocks, group, ilv).splitlines()]
+    ipg = m_blocks * group
+    done = [(g, i) for _, g, i in rows if g >= 0]
+    assert sorted(done) == [(g, i) for g in range(groups) for i in range(ipg)]
+    whole = groups // 8 * 8
+    for bid, g, _ in rows:
+        assert g < 0 or g >= whole or g % 8 == bid % 8
+    # the dispatcher deals an XCD's workgroups to four shader engines in turn: every engine gets
+    # its share of every whole-round group (within the partial turns at the ends of a chunk)
+    for x in range(8):
+        share = Counter((g, (bid // 8) % 4) for bid, g, _ in rows if g >= 0 and g < whole and bid % 8 == x)
+        for g in {g for g, _ in share}:
+            counts = [share[g, e] for e in range(4)]
+            assert max(counts) - min(counts) <= 2, (x, g, counts)
+    # the groups past the whole rounds: ilv at a time, item by item, longest first
+    tail = [(g - whole, i) for _, g, i in sorted(rows, key=lambda r: r[0]) if g >= whole]
+    for c in range(0, groups - whole, ilv):
+        chunk = [i for g, i in tail if c <= g < c + ilv]
+        kc = min(ilv, groups - whole - c)
+        # rotations move a position by less than one turn of the four engines on 8 XCDs
+        assert all(abs(i - w // kc) <= 32 // kc + 1 for w, i in enumerate(chunk))

@@ -42,7 +42,9 @@ __host__ __device__ __forceinline__ int fast_div(int n, const FastDiv& f) {
 //     every block of the last group, which shortens the launch's tail, as
 //     long as ilv groups' K/V stay in the XCD's L2 (interleave_groups);
 //   * for the last G % 8 groups: their items dealt over all 8 XCDs (position
-//     8 j' + x), which also covers a launch with fewer than 8 groups.
+//     8 j' + x), which also covers a launch with fewer than 8 groups.  Those
+//     groups run ilv at a time as well, so that such a launch, too, starts with
+//     the long query blocks of several groups and ends on the short ones.
 // per_xcd (the grid is 8 * per_xcd) = (G / 8) * ipg + ceil((G % 8) * ipg / 8).
 __host__ __device__ inline int64_t work_items_per_xcd(int64_t groups, int64_t ipg) {
   return (groups / 8) * ipg + ((groups % 8) * ipg + 7) / 8;
@@ -54,7 +56,7 @@ struct WorkMap {
   int tail;     // groups after the whole rounds
   int full_j;  // workgroups per XCD in whole rounds
   int per_xcd;  // workgroups per XCD
-  FastDiv by_chunk, by_ilv, by_last, by_ipg;  // ilv ipg, ilv, kc of the last chunk, ipg
+  FastDiv by_chunk, by_ilv, by_last, by_last_tail;  // ilv ipg, ilv, kc of the last chunks
   FastDiv by_group, by_hk;                          // query heads per KV head, KV heads
 };
 inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int hk) {
@@ -69,10 +71,27 @@ inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int h
   w.by_chunk = make_fast_div(chunk < INT32_MAX ? (int)chunk : INT32_MAX);
   w.by_ilv = make_fast_div(ilv);
   w.by_last = make_fast_div(w.gpx % ilv != 0 ? w.gpx % ilv : ilv);
-  w.by_ipg = make_fast_div(ipg);
+  w.by_last_tail = make_fast_div(w.tail % ilv != 0 ? w.tail % ilv : ilv);
   w.by_group = make_fast_div(group);
   w.by_hk = make_fast_div(hk);
   return w;
+}
+// The order in which an XCD's workgroups take the mapping's positions.  The
+// dispatcher deals an XCD's workgroups to its four shader engines in turn, busy or
+// not, so an order with a period of 2 or 4 (groups interleaved 2 or 4 at a time,
+// heads in groups of 4, query blocks of falling length) gives one engine all of one
+// group's or the longest items: with sequences of different lengths it works on
+// while the others idle.  Positions 4q .. 4q + 3 are therefore rotated by q.  Packed
+// prompts of 32/8 heads, head_dim 128, call in us: 8 of 479 .. 1837 tokens with int8 V 229 ->
+// 168, 8 of 200 .. 2000 235 -> 150, 16 of 400 .. 4000 969 -> 804; equal lengths 0 to 1% either way.
+// Periods of 8 and 16 measured 174 / 152 / 797 and 182 / 159 / 803.
+__host__ __device__ __forceinline__ int spread_workgroup(const WorkMap& w, int bid) {
+  const int x = bid & 7, j = bid >> 3;
+  const int base = j < w.full_j ? 0 : w.full_j, n = j < w.full_j ? w.full_j : w.per_xcd - w.full_j;
+  int p = j - base;
+  const int q = p >> 2;
+  if (4 * q + 4 <= n) p = 4 * q + ((p + q) & 3);
+  return (base + p) * 8 + x;
 }
 // The group of workgroup `bid` and its item in the group; false: no item.
 __host__ __device__ __forceinline__ bool work_position(const WorkMap& w, int bid, int& grp, int& item) {
@@ -87,9 +106,12 @@ __host__ __device__ __forceinline__ bool work_position(const WorkMap& w, int bid
     return true;
   }
   const int n = 8 * (j - w.full_j) + x;
-  grp = fast_div(n, w.by_ipg);
-  item = n - grp * w.ipg;
-  grp += 8 * w.gpx;
+  const int c = fast_div(n, w.by_chunk);
+  const int p = n - c * w.by_chunk.d;
+  const bool last = w.tail - c * w.ilv < w.ilv;
+  const FastDiv by_kc = last ? w.by_last_tail : w.by_ilv;
+  item = fast_div(p, by_kc);
+  grp = 8 * w.gpx + c * w.ilv + p - item * by_kc.d;
   return n < w.tail * w.ipg;
 }
 // The same as an item number, or -1.
@@ -157,12 +179,11 @@ __device__ __forceinline__ RowSpan scale_span(const int32_t* cu, int uni, int ro
   return RowSpan{cu[z], cu[z + 1]};
 }
 
-// Groups interleaved per XCD (work_item): as many as keep their K/V tiles
+// Groups interleaved per XCD (work_position): as many as keep their K/V tiles
 // (fp16 K and V, int8 K: 5 bytes per key and head-dim column) within ~5.5 MB,
-// a little over one XCD's 4 MB L2, at most 4.  Measured on cfg2-like
-// launches: 4096 keys (2.6 MB per group) -> 2, 2048 keys -> 4 (-2.6% / -4.3%
-// kernel time); 8192-key groups stay at 1 (2 or 4 of them thrash the L2:
-// +15% / +46%).
+// a little over one XCD's 4 MB L2, at most 4.  Call in us at 1 / 2 / 3 / 4:
+// 8 x 2048 (2048 keys -> 4) 272 / 265 / 265 / 260, 8 x 4096 (2.6 MB per group -> 2) 827 /
+// 804 / 801 / 805, 24 packed prompts of up to 8031 tokens (-> 1) 3591 / 3615 / 3657 / 3655.
 __host__ __device__ inline int interleave_groups(int64_t max_seqlen_k, int head_dim) {
   const int64_t group_bytes = max_seqlen_k * (int64_t)head_dim * 5;
   const int64_t k = group_bytes > 0 ? (int64_t)(5632 * 1024) / group_bytes : 4;

@@ -82,7 +82,7 @@ attn16_kernel(const AttnKArgs a) {
 
   // ---- work item ---------------------------------------------------------
   int grp, item;
-  if (!work_position(a.work, blockIdx.x, grp, item)) return;
+  if (!work_position(a.work, spread_workgroup(a.work, blockIdx.x), grp, item)) return;
   const int mrev = fast_div(item, a.work.by_group), g = item - mrev * a.group;
   const int z = fast_div(grp, a.work.by_hk), hk = grp - z * a.hk;
   const int m = a.m_blocks - 1 - mrev;
