@@ -45,6 +45,9 @@ def test_launch_order(dump_bin, groups, m_blocks, group, ilv):
     whole = groups // 8 * 8
     for bid, g, _ in rows:
         assert g < 0 or g >= whole or g % 8 == bid % 8
+    per_xcd = len(rows) // 8
+    if 32 < per_xcd <= 64:
+        return  # every workgroup starts at once: test_two_workgroups_per_cu
     # the dispatcher deals an XCD's workgroups to four shader engines in turn: every engine gets
     # its share of every whole-round group (within the partial turns at the ends of a chunk)
     for x in range(8):
@@ -59,3 +62,18 @@ def test_launch_order(dump_bin, groups, m_blocks, group, ilv):
         kc = min(ilv, groups - whole - c)
         # rotations move a position by less than one turn of the four engines on 8 XCDs
         assert all(abs(i - w // kc) <= 32 // kc + 1 for w, i in enumerate(chunk))
+
+
+@pytest.mark.parametrize("groups,m_blocks,group", [(8, 11, 3), (8, 16, 3), (8, 16, 4), (16, 8, 3), (8, 33, 1)])
+def test_two_workgroups_per_cu(dump_bin, groups, m_blocks, group):
+    """33 to 64 workgroups per XCD, item 0 the longest query block: workgroup j + 32 shares the CU
+    of workgroup j.  The longest items are alone; of the others, longest goes with shortest."""
+    rows = [tuple(map(int, ln.split())) for ln in _run(dump_bin, groups, m_blocks, group, 4).splitlines()]
+    n = len(rows) // 8
+    assert 32 < n <= 64
+    for x in range(8):
+        rank = sorted(range(n), key=lambda j: (rows[8 * j + x][2], rows[8 * j + x][1]))  # positions, longest first
+        at = {j: r for r, j in enumerate(rank)}
+        alone = [at[j] for j in range(n - 32, 32)]
+        assert alone == list(range(64 - n))
+        assert all(at[j] + at[j + 32] == 63 for j in range(n - 32))

@@ -85,12 +85,26 @@ inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int h
 // prompts of 32/8 heads, head_dim 128, call in us: 8 of 479 .. 1837 tokens with int8 V 229 ->
 // 168, 8 of 200 .. 2000 235 -> 150, 16 of 400 .. 4000 969 -> 804; equal lengths 0 to 1% either way.
 // Periods of 8 and 16 measured 174 / 152 / 797 and 182 / 159 / 803.
+//
+// With more workgroups than an XCD has CUs, but no more than two each, all of them
+// start at once, one per CU first (workgroup j + 32 shares the CU of workgroup j), and
+// a pair shares its SIMDs to the end.  Of n = 32 + k items the longest 32 - k then get
+// a CU to themselves, and the k next ones are paired with the k shortest, longest
+// with shortest.  Against longest first throughout (us, K quantisation included): 24/8
+// heads 1 x 1537 38.7 -> 37.1, 1 x 2048 51.0 -> 48.0 (fp16 mode 46.2 -> 42.9), 3 x 700
+// 28.7 -> 27.1; 28/4 heads 1 x 1537 40.6 -> 38.6, 1 x 2200 58.2 -> 55.4.
+constexpr int kXcdCus = 32;
 __host__ __device__ __forceinline__ int spread_workgroup(const WorkMap& w, int bid) {
   const int x = bid & 7, j = bid >> 3;
   const int base = j < w.full_j ? 0 : w.full_j, n = j < w.full_j ? w.full_j : w.per_xcd - w.full_j;
   int p = j - base;
   const int q = p >> 2;
-  if (4 * q + 4 <= n) p = 4 * q + ((p + q) & 3);
+  if (n == w.per_xcd && n > kXcdCus && n <= 2 * kXcdCus) {
+    const int k = n - kXcdCus;
+    p = p < k ? kXcdCus - k + p : p < kXcdCus ? p - k : n - 1 - (p - kXcdCus);
+  } else if (4 * q + 4 <= n) {
+    p = 4 * q + ((p + q) & 3);
+  }
   return (base + p) * 8 + x;
 }
 // The group of workgroup `bid` and its item in the group; false: no item.
