@@ -240,6 +240,27 @@ __device__ __forceinline__ uint32_t pk_max3(uint32_t x, uint32_t y, uint32_t z) 
   return r;
 }
 
+// The larger half of a packed fp16 pair, as fp32.
+__device__ __forceinline__ float pk_larger(uint32_t x) {
+  uint32_t r;
+  asm("v_pk_max_f16 %0, %1, %1 op_sel:[1,0]" : "=v"(r) : "v"(x));
+  return (float)__builtin_bit_cast(f16x2, r)[0];
+}
+
+// fp32 maximum / minimum without the operand canonicalisation of fmaxf / fminf
+// (the operands are results of arithmetic: never signalling NaNs; a NaN loses to
+// the other operand, as in fmaxf / fminf).
+__device__ __forceinline__ float max_raw(float x, float y) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+  return r;
+}
+__device__ __forceinline__ float min_raw(float x, float y) {
+  float r;
+  asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+  return r;
+}
+
 // Eight int8 codes (bytes of w[0], then w[1]) to fp16, exactly: with the
 // sign bit flipped a code b is the byte u = b + 128, the fp16 with bits
 // 0x64XX is 1024 + u, and 1024 + u - 1152 = b (all exact small integers).

@@ -744,11 +744,15 @@ attn32_kernel(const AttnKArgs a) {
     const uint32_t u0 = pk_max3(s16[0][0], s16[0][1], s16[0][2]), u1 = pk_max3(s16[0][3], s16[0][4], s16[0][5]);
     const uint32_t u2 = pk_max3(s16[0][6], s16[0][7], s16[1][0]), u3 = pk_max3(s16[1][1], s16[1][2], s16[1][3]);
     const uint32_t u4 = pk_max3(s16[1][4], s16[1][5], s16[1][6]);
-    const f16x2 mx2 = __builtin_bit_cast(f16x2, pk_max(pk_max3(u0, u1, u2), pk_max3(u3, u4, s16[1][7])));
-    const float mx = fmaxf((float)mx2[0], (float)mx2[1]);
-    const float2 sw = swap_halves(mx);
-    return fmaxf(sw.x, sw.y);
+    const float2 sw = swap_halves(pk_larger(pk_max(pk_max3(u0, u1, u2), pk_max3(u3, u4, s16[1][7]))));
+    return max_raw(sw.x, sw.y);
   };
+  // (The plain C++ forms of these maxima and of the update below cost 8 more VALU
+  // instructions and 4 wait states per tile in canonicalisations, compares and
+  // selects: B8 x 2048, 32/8 heads, head_dim 64 192.1 -> 190.0 us, int8 V 215.3 -> 211.5.)
+  // exp2(m - max(m, mx)) as exp2(min(m - mx, 0)): 1 when the step brings nothing new,
+  // also while no key has been valid (m = mx = -inf: the NaN loses to 0).
+  auto rescale_of = [&](float mx) -> float { return fast_exp2(min_raw(m_i - mx, 0.0f)); };
 
   // ---- online softmax update (reference _softmax_prefix_update) ------------
   // m_next is the row's new maximum, alpha = exp2(m_i - m_next) (1 if the
@@ -756,8 +760,9 @@ attn32_kernel(const AttnKArgs a) {
   // rescaled by alpha, O^T += V^T . P^T.  svc: the tile's V scales (int8 V).
   auto tile_update = [&](const unsigned char* stage, int route, const f16 (&svc)[NSG],
                          const uint32_t (&s16)[2][8], float m_next, float alpha) {
-    // With no valid key yet the tile is all -inf and p must be 0: subtract 0.
-    const float negm = m_next == -INFINITY ? 0.0f : -m_next;
+    // With no valid key yet the tile is all -inf and p must be 0: -m is clamped to
+    // the largest finite value, and exp2(-inf + FLT_MAX) = 0.
+    const float negm = min_raw(-m_next, 3.40282347e38f);
     // P^T as the B operands of the PV MFMAs: pv[ks] holds keys 16 ks .. 16 ks + 15
     // of this lane's slots (pairs (kb, j) with ks = 2 kb + j / 4).
     u32x4 pv[4];
@@ -983,10 +988,7 @@ attn32_kernel(const AttnKArgs a) {
         issue_next(n + 1, smem_lds + ((n + 1) & 1) * STAGE, route_next, sk_next, sv_next);
       tile_mask(key0, s16);
       const float mx = tile_max(s16);
-      const bool has = mx != -INFINITY;
-      const float m_next = has ? fmaxf(m_i, mx) : m_i;
-      const float alpha = has ? fast_exp2(m_i - m_next) : 1.0f;
-      tile_update(stage, route, svc, s16, m_next, alpha);
+      tile_update(stage, route, svc, s16, max_raw(m_i, mx), rescale_of(mx));
     }
     for (int n = max(n_wave, n_sw); n < n_blocks; ++n) tile_start(n);
   } else {
@@ -1012,18 +1014,16 @@ attn32_kernel(const AttnKArgs a) {
         tile_mask(key0, s16);
         const float mx = tile_max(s16);
         if (cur.pass == 0) {
-          gmx = fmaxf(gmx, mx);
+          gmx = max_raw(gmx, mx);
         } else {
           // The group's maximum enters at its first tile (alpha once per
           // block_n tile); later tiles of the group keep m (alpha = 1).
           float m_next = m_i, alpha = 1.0f;
           if (cur.n == cur.gs) {
-            const float gm = fmaxf(gmx, mx);
+            const float gm = max_raw(gmx, mx);
             gmx = -INFINITY;
-            if (gm != -INFINITY) {
-              m_next = fmaxf(m_i, gm);
-              alpha = fast_exp2(m_i - m_next);
-            }
+            m_next = max_raw(m_i, gm);
+            alpha = rescale_of(gm);
           }
           tile_update(stage, route, svc, s16, m_next, alpha);
         }
