@@ -49,6 +49,7 @@ __host__ __device__ __forceinline__ int fast_div(int n, const FastDiv& f) {
 __host__ __device__ inline int64_t work_items_per_xcd(int64_t groups, int64_t ipg) {
   return (groups / 8) * ipg + ((groups % 8) * ipg + 7) / 8;
 }
+constexpr int kXcdCus = 32;
 // The mapping's constants, computed once per launch on the host.
 struct WorkMap {
   int ipg, ilv;
@@ -56,10 +57,11 @@ struct WorkMap {
   int tail;     // groups after the whole rounds
   int full_j;  // workgroups per XCD in whole rounds
   int per_xcd;  // workgroups per XCD
+  int pair;     // one to two workgroups per CU, of falling length: paired (spread_workgroup)
   FastDiv by_chunk, by_ilv, by_last, by_last_tail;  // ilv ipg, ilv, kc of the last chunks
   FastDiv by_group, by_hk;                          // query heads per KV head, KV heads
 };
-inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int hk) {
+inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int hk, bool causal = true) {
   WorkMap w;
   w.ipg = ipg;
   w.ilv = ilv;
@@ -67,6 +69,7 @@ inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int h
   w.tail = total_items / ipg % 8;
   w.full_j = w.gpx * ipg;
   w.per_xcd = (int)work_items_per_xcd(total_items / ipg, ipg);
+  w.pair = causal && w.per_xcd > kXcdCus && w.per_xcd <= 2 * kXcdCus && (w.full_j == 0 || w.tail == 0);
   const int64_t chunk = (int64_t)ilv * ipg;
   w.by_chunk = make_fast_div(chunk < INT32_MAX ? (int)chunk : INT32_MAX);
   w.by_ilv = make_fast_div(ilv);
@@ -88,18 +91,18 @@ inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int h
 //
 // With more workgroups than an XCD has CUs, but no more than two each, all of them
 // start at once, one per CU first (workgroup j + 32 shares the CU of workgroup j), and
-// a pair shares its SIMDs to the end.  Of n = 32 + k items the longest 32 - k then get
+// a pair shares its SIMDs to the end.  (Causal launches: without the causal limit all
+// items are equally long.)  Of n = 32 + k items the longest 32 - k then get
 // a CU to themselves, and the k next ones are paired with the k shortest, longest
 // with shortest.  Against longest first throughout (us, K quantisation included): 24/8
 // heads 1 x 1537 38.7 -> 37.1, 1 x 2048 51.0 -> 48.0 (fp16 mode 46.2 -> 42.9), 3 x 700
 // 28.7 -> 27.1; 28/4 heads 1 x 1537 40.6 -> 38.6, 1 x 2200 58.2 -> 55.4.
-constexpr int kXcdCus = 32;
 __host__ __device__ __forceinline__ int spread_workgroup(const WorkMap& w, int bid) {
   const int x = bid & 7, j = bid >> 3;
   const int base = j < w.full_j ? 0 : w.full_j, n = j < w.full_j ? w.full_j : w.per_xcd - w.full_j;
   int p = j - base;
   const int q = p >> 2;
-  if (n == w.per_xcd && n > kXcdCus && n <= 2 * kXcdCus) {
+  if (w.pair) {
     const int k = n - kXcdCus;
     p = p < k ? kXcdCus - k + p : p < kXcdCus ? p - k : n - 1 - (p - kXcdCus);
   } else if (4 * q + 4 <= n) {
