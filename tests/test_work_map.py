@@ -77,3 +77,19 @@ def test_two_workgroups_per_cu(dump_bin, groups, m_blocks, group):
         alone = [at[j] for j in range(n - 32, 32)]
         assert alone == list(range(64 - n))
         assert all(at[j] + at[j + 32] == 63 for j in range(n - 32))
+
+
+@pytest.mark.parametrize("groups,m_blocks,group", [(8, 65, 1), (8, 24, 4), (8, 18, 4), (16, 15, 3), (8, 13, 5)])
+def test_three_workgroups_per_cu(dump_bin, groups, m_blocks, group):
+    """65 to 96 workgroups per XCD of which a CU holds three: every item once, and workgroup j + 32,
+    on the CU of workgroup j, is the shorter the longer that is; the rest stays longest first."""
+    rows = [tuple(map(int, ln.split())) for ln in _run(dump_bin, groups, m_blocks, group, 4, 3).splitlines()]
+    n = len(rows) // 8
+    assert 64 < n <= 96
+    assert sorted((g, i) for _, g, i in rows) == [(g, i) for g in range(groups) for i in range(m_blocks * group)]
+    for x in range(8):
+        rank = sorted(range(n), key=lambda j: (rows[8 * j + x][2], rows[8 * j + x][1]))
+        at = {j: r for r, j in enumerate(rank)}
+        assert all(at[j] == j for j in range(32))
+        assert all(at[j + 32] == 63 - j for j in range(32))
+        assert all(at[j] == j for j in range(64, n))

@@ -233,7 +233,8 @@ int launch_attn(const tilemix_attn_params& p, int uniform_seqlen, int32_t* dump_
     const char* env = getenv("TILEMIX_HIP_INTERLEAVE");
     if (env != nullptr && env[0] >= '1' && env[0] <= '4' && env[1] == '\0') ilv = env[0] - '0';
   }
-  a.work = make_work_map((int)total, m_blocks * a.group, ilv, a.group, p.heads_k, p.causal != 0);
+  a.work = make_work_map((int)total, m_blocks * a.group, ilv, a.group, p.heads_k, p.causal != 0,
+                         p.head_dim <= 64 ? 3 : 2);
 
   const int dp = p.head_dim <= 64 ? 64 : 128;
   dispatch_attn(a, kind, dp, p.routing_mode, int8v, dump, p.bias != nullptr, gen, stream);

@@ -49,19 +49,20 @@ __host__ __device__ __forceinline__ int fast_div(int n, const FastDiv& f) {
 __host__ __device__ inline int64_t work_items_per_xcd(int64_t groups, int64_t ipg) {
   return (groups / 8) * ipg + ((groups % 8) * ipg + 7) / 8;
 }
-constexpr int kXcdCus = 32;
+constexpr int kXcdCus = 32;  // CUs per XCD
 // The mapping's constants, computed once per launch on the host.
 struct WorkMap {
   int ipg, ilv;
   int gpx;      // whole-round groups per XCD
   int tail;     // groups after the whole rounds
-  int full_j;  // workgroups per XCD in whole rounds
+  int full_j;   // workgroups per XCD in whole rounds
   int per_xcd;  // workgroups per XCD
-  int pair;     // one to two workgroups per CU, of falling length: paired (spread_workgroup)
+  int share;    // workgroups that share a CU from the start, of falling length (spread_workgroup): 2, 3 or 0
   FastDiv by_chunk, by_ilv, by_last, by_last_tail;  // ilv ipg, ilv, kc of the last chunks
   FastDiv by_group, by_hk;                          // query heads per KV head, KV heads
 };
-inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int hk, bool causal = true) {
+inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int hk, bool causal = true,
+                             int wgs_per_cu = 2) {
   WorkMap w;
   w.ipg = ipg;
   w.ilv = ilv;
@@ -69,7 +70,8 @@ inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int h
   w.tail = total_items / ipg % 8;
   w.full_j = w.gpx * ipg;
   w.per_xcd = (int)work_items_per_xcd(total_items / ipg, ipg);
-  w.pair = causal && w.per_xcd > kXcdCus && w.per_xcd <= 2 * kXcdCus && (w.full_j == 0 || w.tail == 0);
+  const int share = (w.per_xcd + kXcdCus - 1) / kXcdCus;
+  w.share = causal && share >= 2 && share <= wgs_per_cu && share <= 3 && (w.full_j == 0 || w.tail == 0) ? share : 0;
   const int64_t chunk = (int64_t)ilv * ipg;
   w.by_chunk = make_fast_div(chunk < INT32_MAX ? (int)chunk : INT32_MAX);
   w.by_ilv = make_fast_div(ilv);
@@ -97,14 +99,23 @@ inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int h
 // with shortest.  Against longest first throughout (us, K quantisation included): 24/8
 // heads 1 x 1537 38.7 -> 37.1, 1 x 2048 51.0 -> 48.0 (fp16 mode 46.2 -> 42.9), 3 x 700
 // 28.7 -> 27.1; 28/4 heads 1 x 1537 40.6 -> 38.6, 1 x 2200 58.2 -> 55.4.
+//
+// At head_dim <= 64 a CU holds three workgroups, and with 65 to 96 per XCD all start
+// at once as well, by threes (j, j + 32, j + 64).  The longest 32 keep their places,
+// the next 32 run in the opposite order, the rest follows.  Against the rotation (us,
+// causal, head_dim 64, 32/8 heads; the repeats differ by up to 0.6): fp16 mode 1 x 2200
+// 39.4 -> 37.2, 1 x 2600 47.1 -> 42.4, 1 x 3072 59.5 -> 54.2; mixed mode 1 x 2600
+// 56.2 -> 55.8, 1 x 3072 69.3 -> 69.5; 14/2 heads 1 x 5000 100.0 -> 98.1.
 __host__ __device__ __forceinline__ int spread_workgroup(const WorkMap& w, int bid) {
   const int x = bid & 7, j = bid >> 3;
   const int base = j < w.full_j ? 0 : w.full_j, n = j < w.full_j ? w.full_j : w.per_xcd - w.full_j;
   int p = j - base;
   const int q = p >> 2;
-  if (w.pair) {
+  if (w.share == 2) {
     const int k = n - kXcdCus;
     p = p < k ? kXcdCus - k + p : p < kXcdCus ? p - k : n - 1 - (p - kXcdCus);
+  } else if (w.share == 3) {
+    p = p < kXcdCus || p >= 2 * kXcdCus ? p : 3 * kXcdCus - 1 - p;
   } else if (4 * q + 4 <= n) {
     p = 4 * q + ((p + q) & 3);
   }
@@ -131,7 +142,7 @@ __host__ __device__ __forceinline__ bool work_position(const WorkMap& w, int bid
   grp = 8 * w.gpx + c * w.ilv + p - item * by_kc.d;
   return n < w.tail * w.ipg;
 }
-// The same as an item number, or -1.
+// The same as an item number, or -1 (host: the mapping's test).
 inline int work_item(int bid, int total_items, int ipg, int ilv) {
   const WorkMap w = make_work_map(total_items, ipg, ilv, 1, 1);
   int grp, item;

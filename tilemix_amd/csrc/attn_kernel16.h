@@ -37,7 +37,7 @@
 //     pattern of the MFMA operands bank-conflict free;
 //   * INT8 tiles accumulate on top of a magic bias (1.5*2^23 as int bits) so
 //     the exact fp32(acc)*ss of the reference is one FMA;
-//   * blockIdx -> work mapping is XCD-aware (work_item in attn_common.h):
+//   * blockIdx -> work mapping is XCD-aware (work_position in attn_common.h):
 //     whole (sequence, kv-head) groups are dealt round-robin to the 8 XCDs, so
 //     the query heads that share K/V (GQA) and all query blocks of a head hit
 //     the same L2 and every XCD gets the same mix of sequence lengths; within a
