@@ -95,7 +95,8 @@ int tilemix_quant_per_block_int8(const tilemix_quant_params* p, void* stream);
  * or all of Q, K and V.  uniform_seqlen > 0: sequence b is tokens
  * [b * uniform_seqlen, (b + 1) * uniform_seqlen) of every tensor; cu_seqlens and
  * max_seqlen are then not read (cu_seqlens may be NULL), and cu_seqlens_scale is
- * written if it is not NULL.  uniform_seqlen = 0: each tensor's own cu_seqlens.
+ * written if it is not NULL; batch * uniform_seqlen must be below 2^31.
+ * uniform_seqlen = 0: each tensor's own cu_seqlens.
  */
 int tilemix_quant_per_block_int8_many(const tilemix_quant_params* p, int32_t count, int32_t uniform_seqlen,
                                       void* stream);
@@ -175,7 +176,7 @@ int tilemix_attn_fwd(const tilemix_attn_params* p, void* stream);
  * sequence z is tokens [z * seqlen, (z + 1) * seqlen), its scale rows start at
  * z * ceil(seqlen / blk).  No cu array is read (all may be NULL), so the caller
  * builds none and the workgroups need not wait for them.  max_seqlen_q and
- * max_seqlen_k must equal seqlen.
+ * max_seqlen_k must equal seqlen; batch * seqlen must be below 2^31.
  */
 int tilemix_attn_fwd_uniform(const tilemix_attn_params* p, int32_t seqlen, void* stream);
 

@@ -45,3 +45,14 @@ def test_several_tensors_validation(lib):
     assert b"share the batch" in lib.tilemix_last_error()
     assert lib.tilemix_quant_per_block_int8_many(q, 1, 0, None) == 1  # no uniform length: cu_seqlens needed
     assert b"null tensor pointer" in lib.tilemix_last_error()
+
+
+def test_uniform_quantisation_token_index(lib):
+    """More tokens than a 32-bit index holds are refused before anything is launched."""
+    p = (_native.QuantParams * 1)()
+    p[0].input = p[0].output = p[0].scale = 16
+    p[0].heads, p[0].head_dim, p[0].blk_tokens = 1, 8, 64
+    for length, batch in ((1 << 16, 1 << 15), (64, 1 << 26), (2**31 - 1, 2)):
+        p[0].batch = batch
+        assert lib.tilemix_quant_per_block_int8_many(p, 1, length, None) == 1
+        assert b"32-bit token index" in lib.tilemix_last_error()

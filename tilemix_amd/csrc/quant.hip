@@ -288,6 +288,12 @@ int launch_quant(const tilemix_quant_params* ps, int count, int uniform_seqlen, 
                 ps[0].batch, p.batch);
       return TILEMIX_E_INVALID;
     }
+    // The kernel numbers tokens in 32 bits (cu_seqlens does so by its type).
+    if ((int64_t)uniform_seqlen * p.batch > INT32_MAX) {
+      set_error("tilemix_quant_per_block_int8: %d sequences of %d tokens exceed the 32-bit token index", p.batch,
+                uniform_seqlen);
+      return TILEMIX_E_INVALID;
+    }
     const int max_seqlen = uniform_seqlen > 0 ? uniform_seqlen : p.max_seqlen;
     // With no tokens, one block per sequence still publishes cu_seqlens_scale.
     const int64_t nblk = std::max<int64_t>(1, ((int64_t)max_seqlen + p.blk_tokens - 1) / p.blk_tokens);
