@@ -82,3 +82,21 @@ def test_uniform_lengths_equal_cu_seqlens(device, length):
     rows = int(cu_scale[-1])
     for a, b, n in zip(got, (codes, scale, scale16, cu_scale), (len(codes), rows, rows, batch + 1)):
         assert torch.equal(a[:n], b[:n])
+
+
+def test_more_blocks_than_one_launch_takes(device):
+    """Blocks of one token: 9 + 17 heads of 2^20 + 3 tokens are more workgroups than a launch has
+    (2^24 of 256 threads), and the 17 heads alone are, too."""
+    n = (1 << 20) + 3
+    cu = torch.tensor([0, n], dtype=torch.int32, device=device)
+    g = torch.Generator(device=device).manual_seed(11)
+    xs = [torch.randn(n, heads, 8, generator=g, device=device).half() for heads in (9, 17)]
+    results, cu_scales = quantize_many([(x, cu, n, 1, 1.0) for x in xs], half_scales=True)
+    torch.cuda.synchronize()
+    assert cu_scales.tolist() == [[0, n], [0, n]]
+    for x, (codes, scale, scale16) in zip(xs, results):
+        amax = x.abs().amax(-1).float()
+        want = amax / torch.full_like(amax, 127.0)  # IEEE quotients: by a Python number torch multiplies by 1/127
+        assert torch.equal(scale[:n], want) and torch.equal(scale16[:n], want.half())
+        t = x.float() / want[..., None]
+        assert torch.equal(codes, torch.trunc(t + torch.where(t >= 0, 0.5, -0.5)).to(torch.int8))

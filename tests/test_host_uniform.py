@@ -56,3 +56,13 @@ def test_uniform_quantisation_token_index(lib):
         p[0].batch = batch
         assert lib.tilemix_quant_per_block_int8_many(p, 1, length, None) == 1
         assert b"32-bit token index" in lib.tilemix_last_error()
+
+
+def test_quantisation_block_limit(lib):
+    """A sequence of 2^24 blocks or more is refused with the limit (HIP launches fewer than 2^32 threads
+    along x); what lies between is launched in pieces."""
+    p = (_native.QuantParams * 1)()
+    p[0].input = p[0].output = p[0].scale = p[0].cu_seqlens = 16
+    p[0].heads, p[0].head_dim, p[0].blk_tokens, p[0].batch, p[0].max_seqlen = 1, 8, 1, 1, 1 << 24
+    assert lib.tilemix_quant_per_block_int8_many(p, 1, 0, None) == 1
+    assert b"at most 16777215 blocks" in lib.tilemix_last_error()

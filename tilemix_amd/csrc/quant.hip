@@ -36,6 +36,8 @@ namespace {
 constexpr int kQuantThreads = 256;
 constexpr int kRegRows = 8;    // row groups a thread holds in registers
 constexpr int kQuantMany = 3;  // tensors per launch
+// Workgroups of a launch along x: HIP takes less than 2^32 threads there.
+constexpr int64_t kQuantGrid = (int64_t(1) << 32) / kQuantThreads - 1;
 
 struct QuantTensor {
   const f16* in;
@@ -48,7 +50,8 @@ struct QuantTensor {
   int64_t capacity;
   float sm_scale;
   int heads, d, blk;
-  int first;  // first workgroup of this tensor within a sequence's
+  int first;      // first workgroup of this tensor within a sequence's
+  int first_blk;  // first block of this launch
 };
 
 struct QuantKArgs {
@@ -92,7 +95,8 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
   if (args.count > 2 && id >= args.t[2].first) a = args.t[2];
   const int uni = args.uni;
   const int t = id - a.first;
-  const int blk = t / a.heads, h = t - blk * a.heads;
+  const int row = t / a.heads, h = t - row * a.heads;
+  const int blk = a.first_blk + row;
   const int b = blockIdx.y;
 
   const int start = uni > 0 ? b * uni : a.cu[b];
@@ -275,10 +279,9 @@ int launch_quant(const tilemix_quant_params* ps, int count, int uniform_seqlen, 
               kQuantMany, count, uniform_seqlen);
     return TILEMIX_E_INVALID;
   }
-  QuantKArgs a;
-  a.count = 0;
+  QuantKArgs a{};
   a.uni = uniform_seqlen;
-  int64_t total = 0;
+  int64_t total = 0, blocks[kQuantMany];
   for (int i = 0; i < count; ++i) {
     const tilemix_quant_params& p = ps[i];
     const int status = check_quant(p, uniform_seqlen > 0);
@@ -297,6 +300,12 @@ int launch_quant(const tilemix_quant_params* ps, int count, int uniform_seqlen, 
     const int max_seqlen = uniform_seqlen > 0 ? uniform_seqlen : p.max_seqlen;
     // With no tokens, one block per sequence still publishes cu_seqlens_scale.
     const int64_t nblk = std::max<int64_t>(1, ((int64_t)max_seqlen + p.blk_tokens - 1) / p.blk_tokens);
+    if (p.batch > 0 && (nblk > kQuantGrid || p.heads > kQuantGrid)) {
+      set_error("tilemix_quant_per_block_int8: at most %lld blocks in a sequence and heads, got %lld and %d",
+                (long long)kQuantGrid, (long long)nblk, p.heads);
+      return TILEMIX_E_INVALID;
+    }
+    blocks[i] = nblk;
     QuantTensor& t = a.t[a.count++];
     t.in = static_cast<const f16*>(p.input);
     t.out = p.output;
@@ -313,21 +322,35 @@ int launch_quant(const tilemix_quant_params* ps, int count, int uniform_seqlen, 
     t.heads = p.heads;
     t.d = p.head_dim;
     t.blk = p.blk_tokens;
-    t.first = (int)total;
+    t.first = (int)std::min<int64_t>(total, INT32_MAX);
+    t.first_blk = 0;
     total += nblk * p.heads;
-    if (total > INT32_MAX) {
-      set_error("tilemix_quant_per_block_int8: too many blocks (%lld)", (long long)total);
-      return TILEMIX_E_INVALID;
-    }
   }
   if (ps[0].batch == 0) return TILEMIX_OK;
-  for (int i = a.count; i < kQuantMany; ++i) a.t[i] = a.t[0];
-  hipLaunchKernelGGL(quant_per_block_int8_kernel, dim3((unsigned)total, (unsigned)ps[0].batch),
-                     dim3(kQuantThreads), 0, stream, a);
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess) {
+  auto launch = [&](const QuantKArgs& args, int64_t groups) -> int {
+    hipLaunchKernelGGL(quant_per_block_int8_kernel, dim3((unsigned)groups, (unsigned)ps[0].batch),
+                       dim3(kQuantThreads), 0, stream, args);
+    const hipError_t err = hipGetLastError();
+    if (err == hipSuccess) return TILEMIX_OK;
     set_error("tilemix_quant_per_block_int8: launch failed: %s", hipGetErrorString(err));
     return TILEMIX_E_LAUNCH;
+  };
+  if (total <= kQuantGrid) {
+    for (int i = a.count; i < kQuantMany; ++i) a.t[i] = a.t[0];
+    return launch(a, total);
+  }
+  // One tensor, and as many of its blocks as a launch takes, at a time.
+  for (int i = 0; i < count; ++i) {
+    QuantKArgs one = a;
+    one.count = 1;
+    one.t[0] = a.t[i];
+    one.t[0].first = 0;
+    const int64_t step = kQuantGrid / a.t[i].heads;
+    for (int64_t first = 0; first < blocks[i]; first += step) {
+      one.t[0].first_blk = (int)first;
+      const int status = launch(one, std::min(step, blocks[i] - first) * a.t[i].heads);
+      if (status != TILEMIX_OK) return status;
+    }
   }
   return TILEMIX_OK;
 }
