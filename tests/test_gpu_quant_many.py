@@ -100,3 +100,13 @@ def test_more_blocks_than_one_launch_takes(device):
         assert torch.equal(scale[:n], want) and torch.equal(scale16[:n], want.half())
         t = x.float() / want[..., None]
         assert torch.equal(codes, torch.trunc(t + torch.where(t >= 0, 0.5, -0.5)).to(torch.int8))
+
+
+@pytest.mark.parametrize("heads,dim,blk", [(1, 8, 1), (3, 24, 1), (5, 64, 3), (24, 128, 4), (7, 256, 16), (2, 136, 17)])
+def test_one_tensor_small_blocks(device, heads, dim, blk):
+    """Many workgroups of few rows, most of the grid empty: one long sequence among short and empty ones."""
+    lengths = [2, 0, 301, 1, blk, 0]
+    x, _, _, cu = packed_inputs(lengths, heads, heads, dim, seed=heads + blk)
+    codes, scale, scale16, cu_scale = quantize_blocks(to_dev(x, device), to_dev(cu, device), 301, blk, half_scales=True)
+    torch.cuda.synchronize()
+    _check(codes, scale, scale16, cu_scale, x, cu, blk)

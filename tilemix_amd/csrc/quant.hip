@@ -24,6 +24,14 @@
 // LDS, the scale-row prefix (and its barrier) before the loads, and ~12 instructions
 // per code: K of 8 x 4096 x 8 heads x 128 25.0 -> 18.5 us (5.5 TB/s), Q of 8 x 4096 x 24
 // x 128 65 -> 49 us (6.1 TB/s), K of 8 x 2048 13.6 -> 10.7 us, of 1 x 1000 5.5 -> 4.1 us.
+//
+// Small blocks, and workgroups past the end of their sequence, last as long as
+// their chain of scalar loads and divisions before the first row (or the exit).  Divisors
+// come as multipliers from the host, a launch of one tensor reads its arguments at
+// once, the maximum takes one barrier.  With the divisions, a tensor chosen after a
+// load and two barriers (us): 8192 tokens x 8 heads x 128 in blocks of 1 101 -> 63, of 4
+// 28.4 -> 18.7, of 64 6.6 -> 5.9; 200 prompts of 5 tokens and one of 8000, blocks of 64
+// 161 -> 49.
 #include "attn_common.h"
 
 #include <algorithm>
@@ -48,16 +56,18 @@ struct QuantTensor {
   int32_t* cu_scale;
   int64_t si_t, si_h, so_t, so_h;
   int64_t capacity;
+  FastDiv by_heads, by_chunks;  // heads, 8-element chunks per row
   float sm_scale;
-  int heads, d, blk;
-  int first;      // first workgroup of this tensor within a sequence's
+  int blk;
+  int rpi;        // rows the workgroup reads per step
+  int uni_rows;   // uni > 0: scale rows per sequence
   int first_blk;  // first block of this launch
 };
 
 struct QuantKArgs {
   QuantTensor t[kQuantMany];
-  int count;
-  int uni;  // > 0: every sequence has this many tokens (cu is not read)
+  int first[kQuantMany];  // first workgroup of each tensor within a sequence's (past the grid: no such tensor)
+  int uni;                // > 0: every sequence has this many tokens (cu is not read)
 };
 
 __device__ __forceinline__ uint32_t pk_max_u16(uint32_t x, uint32_t y) {
@@ -86,28 +96,32 @@ __device__ __forceinline__ int wave_sum_i(int v) {
   return v;
 }
 
+// MANY: several tensors.  (A launch of one reads its arguments without waiting for
+// the choice of the tensor.)
+template <bool MANY>
 __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(const QuantKArgs args) {
-  __shared__ uint32_t red[kQuantThreads / 64];
+  __shared__ uint32_t red[2][kQuantThreads / 64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int id = blockIdx.x;
-  QuantTensor a = args.t[0];
-  if (args.count > 1 && id >= args.t[1].first) a = args.t[1];
-  if (args.count > 2 && id >= args.t[2].first) a = args.t[2];
+  const int id = blockIdx.x, b = blockIdx.y;
+  const int tensor = MANY ? (id >= args.first[1]) + (id >= args.first[2]) : 0;
+  const QuantTensor& a = args.t[tensor];
   const int uni = args.uni;
-  const int t = id - a.first;
-  const int row = t / a.heads, h = t - row * a.heads;
+  const int t = MANY ? id - args.first[tensor] : id;
+  const int row = fast_div(t, a.by_heads), heads = a.by_heads.d, h = t - row * heads;
   const int blk = a.first_blk + row;
-  const int b = blockIdx.y;
 
-  const int start = uni > 0 ? b * uni : a.cu[b];
-  const int len = uni > 0 ? uni : a.cu[b + 1] - start;
+  int start = b * uni, len = uni;
+  if (uni <= 0) {
+    start = a.cu[b];
+    len = a.cu[b + 1] - start;
+  }
   const int rows = min(a.blk, len - blk * a.blk);  // <= 0: no such block in this sequence
 
   // Scale-row base of sequence b (the sum of ceil(L / blk) over the earlier
   // ones), needed by wave 0 only: it stores the scale.  Called after the block's
   // loads have gone out.
   auto scale_base = [&]() -> int {
-    if (uni > 0) return b * ((uni + a.blk - 1) / a.blk);
+    if (uni > 0) return b * a.uni_rows;
     int part = 0;
     for (int bb = lane; bb < b; bb += 64) part += (a.cu[bb + 1] - a.cu[bb] + a.blk - 1) / a.blk;
     return wave_sum_i(part);
@@ -123,11 +137,9 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
     return;
   }
 
-  const int cpr = a.d >> 3;                // 8-element chunks per row
-  const int rpi = kQuantThreads / cpr;     // rows the workgroup reads per step
-  const int r0 = tid / cpr, col = (tid - r0 * cpr) << 3;
-  const bool used = r0 < rpi;              // cpr need not divide the workgroup
-  const int groups = (rows + rpi - 1) / rpi;
+  const int rpi = a.rpi;
+  const int r0 = fast_div(tid, a.by_chunks), col = (tid - r0 * a.by_chunks.d) << 3;
+  const bool used = r0 < rpi;  // the chunks per row need not divide the workgroup
   const int64_t tok0 = (int64_t)start + (int64_t)blk * a.blk;
   const f16* in = a.in + (tok0 + r0) * a.si_t + (int64_t)h * a.si_h + col;
   int8_t* out = a.out + (tok0 + r0) * a.so_t + (int64_t)h * a.so_h + col;
@@ -159,14 +171,13 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
   // patterns without their signs order like the values; RN(x * sm) is monotonic
   // in |x|).  The maximum ignores NaNs, whose patterns lie above infinity's: a
   // block that holds one takes its maximum again from the values below.
-  auto block_max = [&](uint32_t m2) -> uint32_t {
+  auto block_max = [&](uint32_t m2, int pass) -> uint32_t {
     const uint32_t m = wave_max_u32(max(m2 & 0xffffu, m2 >> 16));
+    if (lane == 0) red[pass][wave] = m;
     __syncthreads();
-    if (lane == 0) red[wave] = m;
-    __syncthreads();
-    uint32_t r = red[0];
+    uint32_t r = red[pass][0];
 #pragma unroll
-    for (int w = 1; w < kQuantThreads / 64; ++w) r = max(r, red[w]);
+    for (int w = 1; w < kQuantThreads / 64; ++w) r = max(r, red[pass][w]);
     return r;
   };
   constexpr uint32_t kInf = 0x7c00u;
@@ -191,8 +202,8 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
     if (tid == 0) {
       const int64_t row = (int64_t)base + blk;
       if (row < a.capacity) {
-        a.scale[row * a.heads + h] = s;
-        if (a.scale_half != nullptr) a.scale_half[row * a.heads + h] = (f16)s;
+        a.scale[row * heads + h] = s;
+        if (a.scale_half != nullptr) a.scale_half[row * heads + h] = (f16)s;
       }
     }
     publish(base);
@@ -210,12 +221,12 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
     const int base = wave == 0 ? scale_base() : 0;
 #pragma unroll
     for (int i = 0; i < kN; ++i) m2 = magnitudes(xs[i], m2);
-    uint32_t m = block_max(m2);
+    uint32_t m = block_max(m2, 0);
     if (m > kInf) {
       m2 = 0;
 #pragma unroll
       for (int i = 0; i < kN; ++i) m2 = finite_magnitudes(xs[i], m2);
-      m = block_max(m2);
+      m = block_max(m2, 1);
     }
     const float s = scale_of(m);
     const float rs = s == 0.0f ? 0.0f : 1.0f / s;
@@ -224,20 +235,20 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
       if (used && r0 + i * rpi < rows) encode(xs[i], s, rs, out + i * out_step);
     finish(s, base);
   };
-  if (groups <= kRegRows / 2) {
+  if (rows <= rpi * (kRegRows / 2)) {
     in_registers(std::integral_constant<int, kRegRows / 2>{});
-  } else if (groups <= kRegRows) {
+  } else if (rows <= rpi * kRegRows) {
     in_registers(std::integral_constant<int, kRegRows>{});
   } else {
     uint32_t m2 = 0;
     for (int i = 0; used && r0 + i * rpi < rows; ++i)
       m2 = magnitudes(*reinterpret_cast<const u32x4*>(in + i * in_step), m2);
-    uint32_t m = block_max(m2);
+    uint32_t m = block_max(m2, 0);
     if (m > kInf) {
       m2 = 0;
       for (int i = 0; used && r0 + i * rpi < rows; ++i)
         m2 = finite_magnitudes(*reinterpret_cast<const u32x4*>(in + i * in_step), m2);
-      m = block_max(m2);
+      m = block_max(m2, 1);
     }
     const float s = scale_of(m);
     const float rs = s == 0.0f ? 0.0f : 1.0f / s;
@@ -306,7 +317,7 @@ int launch_quant(const tilemix_quant_params* ps, int count, int uniform_seqlen, 
       return TILEMIX_E_INVALID;
     }
     blocks[i] = nblk;
-    QuantTensor& t = a.t[a.count++];
+    QuantTensor& t = a.t[i];
     t.in = static_cast<const f16*>(p.input);
     t.out = p.output;
     t.scale = p.scale;
@@ -319,36 +330,39 @@ int launch_quant(const tilemix_quant_params* ps, int count, int uniform_seqlen, 
     t.so_h = p.stride_out_head;
     t.capacity = p.scale_rows_capacity;
     t.sm_scale = p.sm_scale;
-    t.heads = p.heads;
-    t.d = p.head_dim;
+    t.by_heads = make_fast_div(p.heads);
+    t.by_chunks = make_fast_div(p.head_dim / 8);
     t.blk = p.blk_tokens;
-    t.first = (int)std::min<int64_t>(total, INT32_MAX);
+    t.rpi = kQuantThreads / (p.head_dim / 8);
+    t.uni_rows = uniform_seqlen > 0 ? (uniform_seqlen - 1) / p.blk_tokens + 1 : 0;
     t.first_blk = 0;
+    a.first[i] = (int)std::min<int64_t>(total, INT32_MAX);
     total += nblk * p.heads;
   }
   if (ps[0].batch == 0) return TILEMIX_OK;
-  auto launch = [&](const QuantKArgs& args, int64_t groups) -> int {
-    hipLaunchKernelGGL(quant_per_block_int8_kernel, dim3((unsigned)groups, (unsigned)ps[0].batch),
-                       dim3(kQuantThreads), 0, stream, args);
+  auto launch = [&](const QuantKArgs& args, int64_t groups, bool many) -> int {
+    const dim3 grid((unsigned)groups, (unsigned)ps[0].batch);
+    if (many)
+      hipLaunchKernelGGL((quant_per_block_int8_kernel<true>), grid, dim3(kQuantThreads), 0, stream, args);
+    else
+      hipLaunchKernelGGL((quant_per_block_int8_kernel<false>), grid, dim3(kQuantThreads), 0, stream, args);
     const hipError_t err = hipGetLastError();
     if (err == hipSuccess) return TILEMIX_OK;
     set_error("tilemix_quant_per_block_int8: launch failed: %s", hipGetErrorString(err));
     return TILEMIX_E_LAUNCH;
   };
   if (total <= kQuantGrid) {
-    for (int i = a.count; i < kQuantMany; ++i) a.t[i] = a.t[0];
-    return launch(a, total);
+    for (int i = count; i < kQuantMany; ++i) a.first[i] = INT32_MAX;
+    return launch(a, total, count > 1);
   }
   // One tensor, and as many of its blocks as a launch takes, at a time.
   for (int i = 0; i < count; ++i) {
     QuantKArgs one = a;
-    one.count = 1;
     one.t[0] = a.t[i];
-    one.t[0].first = 0;
-    const int64_t step = kQuantGrid / a.t[i].heads;
+    const int64_t step = kQuantGrid / ps[i].heads;
     for (int64_t first = 0; first < blocks[i]; first += step) {
       one.t[0].first_blk = (int)first;
-      const int status = launch(one, std::min(step, blocks[i] - first) * a.t[i].heads);
+      const int status = launch(one, std::min(step, blocks[i] - first) * ps[i].heads, false);
       if (status != TILEMIX_OK) return status;
     }
   }
