@@ -110,3 +110,15 @@ def test_one_tensor_small_blocks(device, heads, dim, blk):
     codes, scale, scale16, cu_scale = quantize_blocks(to_dev(x, device), to_dev(cu, device), 301, blk, half_scales=True)
     torch.cuda.synchronize()
     _check(codes, scale, scale16, cu_scale, x, cu, blk)
+
+
+@pytest.mark.parametrize("batch", [1, 64, 65, 257, 1100])
+def test_scale_rows_of_many_sequences(device, batch):
+    """The scale-row base is summed by four waves, 64 earlier sequences each at a time."""
+    rng = np.random.default_rng(batch)
+    lengths = rng.integers(0, 9, batch).tolist()
+    lengths[-1] = 5
+    x, _, _, cu = packed_inputs(lengths, 2, 2, 8, seed=batch)
+    codes, scale, scale16, cu_scale = quantize_blocks(to_dev(x, device), to_dev(cu, device), 8, 3, half_scales=True)
+    torch.cuda.synchronize()
+    _check(codes, scale, scale16, cu_scale, x, cu, 3)

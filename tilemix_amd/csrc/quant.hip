@@ -56,9 +56,8 @@ struct QuantTensor {
   int32_t* cu_scale;
   int64_t si_t, si_h, so_t, so_h;
   int64_t capacity;
-  FastDiv by_heads, by_chunks;  // heads, 8-element chunks per row
+  FastDiv by_heads, by_chunks, by_blk;  // heads, 8-element chunks per row, tokens per block
   float sm_scale;
-  int blk;
   int rpi;        // rows the workgroup reads per step
   int uni_rows;   // uni > 0: scale rows per sequence
   int first_blk;  // first block of this launch
@@ -101,6 +100,7 @@ __device__ __forceinline__ int wave_sum_i(int v) {
 template <bool MANY>
 __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(const QuantKArgs args) {
   __shared__ uint32_t red[2][kQuantThreads / 64];
+  __shared__ int red_rows[kQuantThreads / 64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int id = blockIdx.x, b = blockIdx.y;
   const int tensor = MANY ? (id >= args.first[1]) + (id >= args.first[2]) : 0;
@@ -115,32 +115,52 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
     start = a.cu[b];
     len = a.cu[b + 1] - start;
   }
-  const int rows = min(a.blk, len - blk * a.blk);  // <= 0: no such block in this sequence
+  const int blk_tokens = a.by_blk.d;
+  const int rows = min(blk_tokens, len - blk * blk_tokens);  // <= 0: no such block in this sequence
 
-  // Scale-row base of sequence b (the sum of ceil(L / blk) over the earlier
-  // ones), needed by wave 0 only: it stores the scale.  Called after the block's
-  // loads have gone out.
-  auto scale_base = [&]() -> int {
-    if (uni > 0) return b * a.uni_rows;
+  // Scale-row base of sequence b (the sum of ceil(L / blk) over the earlier ones):
+  // each wave's part goes to LDS after the block's loads have gone out, and the thread
+  // that stores the scale adds them behind the maximum's barrier.  The sum is a chain
+  // of loads, so all four waves share it and each keeps four loads in flight: by one
+  // wave alone, a load at a time, 4096 sequences of 16 tokens x 8 heads x 128 take 126 us
+  // instead of 81, 8192 of 4 tokens 367 instead of 187.
+  auto scale_rows = [&](int n) { return n > 0 ? fast_div(n - 1, a.by_blk) + 1 : 0; };
+  auto sum_scale_rows = [&]() {
+    if (uni > 0) return;
     int part = 0;
-    for (int bb = lane; bb < b; bb += 64) part += (a.cu[bb + 1] - a.cu[bb] + a.blk - 1) / a.blk;
-    return wave_sum_i(part);
+    if (b > wave * 64) {
+#pragma unroll 4
+      for (int bb = tid; bb < b; bb += kQuantThreads) part += scale_rows(a.cu[bb + 1] - a.cu[bb]);
+      part = wave_sum_i(part);
+    }
+    if (lane == 0) red_rows[wave] = part;
+  };
+  auto scale_base = [&]() -> int {  // behind a barrier after sum_scale_rows
+    if (uni > 0) return b * a.uni_rows;
+    int base = 0;
+#pragma unroll
+    for (int w = 0; w < kQuantThreads / 64; ++w) base += red_rows[w];
+    return base;
   };
   auto publish = [&](int base) {
-    if (blk == 0 && h == 0 && tid == 0 && a.cu_scale != nullptr) {
-      a.cu_scale[b + 1] = base + (len + a.blk - 1) / a.blk;
+    if (blk == 0 && h == 0 && a.cu_scale != nullptr) {
+      a.cu_scale[b + 1] = base + scale_rows(len);
       if (b == 0) a.cu_scale[0] = 0;
     }
   };
   if (rows <= 0) {
-    if (blk == 0 && h == 0 && wave == 0) publish(scale_base());
+    if (blk == 0 && h == 0) {
+      sum_scale_rows();
+      __syncthreads();
+      if (tid == 0) publish(scale_base());
+    }
     return;
   }
 
   const int rpi = a.rpi;
   const int r0 = fast_div(tid, a.by_chunks), col = (tid - r0 * a.by_chunks.d) << 3;
   const bool used = r0 < rpi;  // the chunks per row need not divide the workgroup
-  const int64_t tok0 = (int64_t)start + (int64_t)blk * a.blk;
+  const int64_t tok0 = (int64_t)start + (int64_t)blk * blk_tokens;
   const f16* in = a.in + (tok0 + r0) * a.si_t + (int64_t)h * a.si_h + col;
   int8_t* out = a.out + (tok0 + r0) * a.so_t + (int64_t)h * a.so_h + col;
   const int64_t in_step = (int64_t)rpi * a.si_t, out_step = (int64_t)rpi * a.so_t;
@@ -198,15 +218,16 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
     const float amax = fmaxf(0.0f, fabsf((float)__builtin_bit_cast(f16, (uint16_t)m) * sm));
     return amax / 127.0f;  // IEEE division (no fast-math in this build)
   };
-  auto finish = [&](float s, int base) {
+  auto finish = [&](float s) {
     if (tid == 0) {
+      const int base = scale_base();
       const int64_t row = (int64_t)base + blk;
       if (row < a.capacity) {
         a.scale[row * heads + h] = s;
         if (a.scale_half != nullptr) a.scale_half[row * heads + h] = (f16)s;
       }
+      publish(base);
     }
-    publish(base);
   };
 
   auto in_registers = [&](auto nreg) {
@@ -218,7 +239,7 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
       xs[i] = (u32x4){};
       if (used && r0 + i * rpi < rows) xs[i] = *reinterpret_cast<const u32x4*>(in + i * in_step);
     }
-    const int base = wave == 0 ? scale_base() : 0;
+    sum_scale_rows();
 #pragma unroll
     for (int i = 0; i < kN; ++i) m2 = magnitudes(xs[i], m2);
     uint32_t m = block_max(m2, 0);
@@ -233,7 +254,7 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
 #pragma unroll
     for (int i = 0; i < kN; ++i)
       if (used && r0 + i * rpi < rows) encode(xs[i], s, rs, out + i * out_step);
-    finish(s, base);
+    finish(s);
   };
   if (rows <= rpi * (kRegRows / 2)) {
     in_registers(std::integral_constant<int, kRegRows / 2>{});
@@ -243,6 +264,7 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
     uint32_t m2 = 0;
     for (int i = 0; used && r0 + i * rpi < rows; ++i)
       m2 = magnitudes(*reinterpret_cast<const u32x4*>(in + i * in_step), m2);
+    sum_scale_rows();
     uint32_t m = block_max(m2, 0);
     if (m > kInf) {
       m2 = 0;
@@ -254,7 +276,7 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
     const float rs = s == 0.0f ? 0.0f : 1.0f / s;
     for (int i = 0; used && r0 + i * rpi < rows; ++i)
       encode(*reinterpret_cast<const u32x4*>(in + i * in_step), s, rs, out + i * out_step);
-    finish(s, wave == 0 ? scale_base() : 0);
+    finish(s);
   }
 }
 
@@ -332,7 +354,7 @@ int launch_quant(const tilemix_quant_params* ps, int count, int uniform_seqlen, 
     t.sm_scale = p.sm_scale;
     t.by_heads = make_fast_div(p.heads);
     t.by_chunks = make_fast_div(p.head_dim / 8);
-    t.blk = p.blk_tokens;
+    t.by_blk = make_fast_div(p.blk_tokens);
     t.rpi = kQuantThreads / (p.head_dim / 8);
     t.uni_rows = uniform_seqlen > 0 ? (uniform_seqlen - 1) / p.blk_tokens + 1 : 0;
     t.first_blk = 0;
