@@ -43,6 +43,10 @@ def test_rms_norm_row_stride_aligned_and_not(device):
     (1, 20, 2, 3, 272),     # fewer than 16 head slots
     (1, 2, 1, 2, 4096),     # one head slot, one token
     (1, 2, 1, 2, 4112),     # past the vector path
+    (1, 1, 1, 1, 128),      # fewer rows than a workgroup takes
+    (3, 4, 1, 13, 64),      # rows that end within a workgroup
+    (1, 20, 4, 11, 80),     # whole tokens per workgroup: 48 of its 51 rows
+    (2, 1, 1, 33, 128),     # two heads; the last workgroup a fraction of a token
 ])
 def test_rotary_shapes_bitexact(device, b, hq, hk, t, d):
     q, k, cos, sin = _rope_inputs(b, hq, hk, t, d, b, seed=d + t, device=device)

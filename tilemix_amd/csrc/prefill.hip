@@ -2,9 +2,11 @@
 // rotary embedding of Q and K, SiLU(gate) * up.  All three are HBM-streaming
 // kernels (one read of every input, one write of every output, 16-byte
 // accesses); the formulas follow models/tilemix_llama.py:718-869.
-#include "common.h"
+#include "attn_common.h"
 
 #include <math.h>
+
+#include <algorithm>
 
 namespace tmx {
 
@@ -125,14 +127,16 @@ __global__ void __launch_bounds__(kNormWaves * 64) rmsnorm_kernel(const NormArgs
 
 // ---- rotary (reference :808-847) -------------------------------------------
 // One thread per pair of 8-element chunks (d, d + D/2) of a (b, t, h) row: the two
-// chunks are each other's rotation partners, so a row is read once.  A thread
-// takes every 16th head (fewer slots for head_dim > 256) of its token with the
-// token's cos / sin chunks in registers.  Output rows are token-major.  Bound by
-// HBM (4 bytes per value) at large token counts, by loads in flight at small ones.
-// Against one thread per chunk that loads its partner chunk too (24 + 8 heads, head_dim
-// 128, us): 2048 tokens 10.8 -> 8.8, 2 x 1537 head-major 13.7 -> 11.9, 32768 tokens 100 ->
-// 101 (5.5 TB/s, a large copy's rate); 8192 tokens of 32 + 8 heads x 64 19.1 -> 16.7.  8 slots:
-// 8.7 / 11.5 / 104 / 16.2; 4 slots: 9.9 / 12.4 / 107 / 19.4.
+// chunks are each other's rotation partners, so a row is read once.  Heads of Q and
+// then K are the fastest row index, so the rows of a token read its cos / sin from
+// cache.  Output rows are token-major.  Bound by HBM (4 bytes per value) at large
+// token counts, by the launch and one round of loads at small ones.
+// Kernel in us, against one thread per chunk that loads its partner chunk too / 16 head
+// slots per token that keep cos / sin over several heads, Q and K in turn (slots
+// idle with few heads, several rounds with many): 24 + 8 heads x 128, 16 tokens 2.63 /
+// 3.53 / 2.41, 2048 9.1 / 7.1 / 6.2, 32768 104 / 98.3 / 95.0 (5.7 TB/s);
+// 4 + 1 heads x 128, 16384 tokens 10.9 / 19.2 / 8.8; 14 + 2 x 64, 2048 3.97 / 4.54 / 3.22.
+// Two, three or four heads per thread with all slots in use were no faster.
 struct RotaryArgs {
   const f16* q;
   const f16* k;
@@ -141,9 +145,11 @@ struct RotaryArgs {
   f16* oq;
   f16* ok;
   int64_t qz, qh, qt, kz, kh, kt, cz, ct, sz, st;
-  int64_t bt;    // batch * tokens
-  int64_t rows;  // bt * (hq + hk)
+  int64_t rows;  // batch * tokens * (hq + hk)
   int t, hq, hk, d;
+  // rotary_kernel: 8-element chunk pairs per row, rows per token, tokens
+  FastDiv by_pairs, by_heads, by_tokens;
+  int per_wg;  // rows of a workgroup, at most 256 / pairs
 };
 
 __device__ __forceinline__ f16 rope_one(float x, float xr, float c, float s, float sign) {
@@ -151,11 +157,6 @@ __device__ __forceinline__ f16 rope_one(float x, float xr, float c, float s, flo
   const f16 b = (f16)((xr * sign) * s);
   return (f16)keep32((float)a + (float)b);
 }
-
-// Workgroup shape for rows of `pairs` chunk pairs: head slots per token (at most 16)
-// and tokens.
-__host__ __device__ inline int rot_heads(int pairs) { return min(16, 256 / pairs); }
-__host__ __device__ inline int rot_tokens(int pairs) { return 256 / pairs / rot_heads(pairs); }
 
 __device__ __forceinline__ f16x8 rope8(const f16x8& x, const f16x8& xr, const f16x8& c, const f16x8& s, float sign) {
   f16x8 o;
@@ -166,57 +167,51 @@ __device__ __forceinline__ f16x8 rope8(const f16x8& x, const f16x8& xr, const f1
 
 __global__ void __launch_bounds__(256) rotary_kernel(const RotaryArgs a) {
   const int half = a.d >> 1;
-  const int cpr = half >> 3;                // chunk pairs per row (d % 16 == 0 on this path)
-  const int heads = rot_heads(cpr), tokens = rot_tokens(cpr);
-  const int slot = threadIdx.x / cpr, d0 = (threadIdx.x - slot * cpr) * 8;
-  const int tl = slot / heads, h0 = slot - tl * heads;
-  const int64_t bt = (int64_t)blockIdx.x * tokens + tl;
-  if (tl >= tokens || bt >= a.bt) return;
-  const int64_t b = bt / a.t, t = bt - b * a.t;
+  const int rl = fast_div(threadIdx.x, a.by_pairs), d0 = (threadIdx.x - rl * a.by_pairs.d) * 8;
+  const int64_t row = (int64_t)blockIdx.x * a.per_wg + rl;
+  if (rl >= a.per_wg || row >= a.rows) return;
+  const int bt = fast_div((int)row, a.by_heads), h = (int)row - bt * a.by_heads.d, hk = h - a.hq;
+  const int b = fast_div(bt, a.by_tokens), t = bt - b * a.t;
   const f16* cs = a.cs + b * a.cz + t * a.ct + d0;
   const f16* sn = a.sn + b * a.sz + t * a.st + d0;
+  const f16* x = (hk < 0 ? a.q + b * a.qz + t * a.qt + h * a.qh : a.k + b * a.kz + t * a.kt + hk * a.kh) + d0;
+  f16* o = (hk < 0 ? a.oq + ((int64_t)bt * a.hq + h) * a.d : a.ok + ((int64_t)bt * a.hk + hk) * a.d) + d0;
   const f16x8 c0 = *reinterpret_cast<const f16x8*>(cs), c1 = *reinterpret_cast<const f16x8*>(cs + half);
   const f16x8 s0 = *reinterpret_cast<const f16x8*>(sn), s1 = *reinterpret_cast<const f16x8*>(sn + half);
-  // Heads h0, h0 + heads, ... of one tensor's n.
-  auto rotate = [&](const f16* src, f16* dst, int n, int64_t head_stride) {
-    for (int h = h0; h < n; h += heads) {
-      const f16* x = src + h * head_stride;
-      const f16x8 x0 = *reinterpret_cast<const f16x8*>(x), x1 = *reinterpret_cast<const f16x8*>(x + half);
-      f16* o = dst + (int64_t)h * a.d;
-      *reinterpret_cast<f16x8*>(o) = rope8(x0, x1, c0, s0, -1.0f);
-      *reinterpret_cast<f16x8*>(o + half) = rope8(x1, x0, c1, s1, 1.0f);
-    }
-  };
-  rotate(a.q + b * a.qz + t * a.qt + d0, a.oq + bt * a.hq * a.d + d0, a.hq, a.qh);
-  rotate(a.k + b * a.kz + t * a.kt + d0, a.ok + bt * a.hk * a.d + d0, a.hk, a.kh);
+  // cos and sin go out first: the other way round 32768 tokens of 32 + 8 heads x 64 take 66.3
+  // instead of 62.8 us.
+  asm volatile("" ::: "memory");
+  const f16x8 x0 = *reinterpret_cast<const f16x8*>(x), x1 = *reinterpret_cast<const f16x8*>(x + half);
+  *reinterpret_cast<f16x8*>(o) = rope8(x0, x1, c0, s0, -1.0f);
+  *reinterpret_cast<f16x8*>(o + half) = rope8(x1, x0, c1, s1, 1.0f);
 }
 
 // Generic element-wise variant (any even head_dim, any alignment).
 __global__ void __launch_bounds__(256) rotary_kernel_scalar(const RotaryArgs a) {
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= a.rows * a.d) return;
-  const int d = (int)(gid % a.d);
-  int64_t r = gid / a.d;
-  const int H = a.hq + a.hk;
-  const int h = (int)(r % H);
-  r /= H;
-  const int t = (int)(r % a.t);
-  const int64_t b = r / a.t;
-  const int half = a.d >> 1;
-  const int dr = (d + half) % a.d;
-  const float sign = d < half ? -1.0f : 1.0f;
-  const f16* src;
-  f16* dst;
-  if (h < a.hq) {
-    src = a.q + b * a.qz + (int64_t)h * a.qh + (int64_t)t * a.qt;
-    dst = a.oq + ((b * a.t + t) * a.hq + h) * a.d;
-  } else {
-    src = a.k + b * a.kz + (int64_t)(h - a.hq) * a.kh + (int64_t)t * a.kt;
-    dst = a.ok + ((b * a.t + t) * a.hk + (h - a.hq)) * a.d;
+  for (int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x; gid < a.rows * a.d; gid += (int64_t)gridDim.x * 256) {
+    const int d = (int)(gid % a.d);
+    int64_t r = gid / a.d;
+    const int H = a.hq + a.hk;
+    const int h = (int)(r % H);
+    r /= H;
+    const int t = (int)(r % a.t);
+    const int64_t b = r / a.t;
+    const int half = a.d >> 1;
+    const int dr = (d + half) % a.d;
+    const float sign = d < half ? -1.0f : 1.0f;
+    const f16* src;
+    f16* dst;
+    if (h < a.hq) {
+      src = a.q + b * a.qz + (int64_t)h * a.qh + (int64_t)t * a.qt;
+      dst = a.oq + ((b * a.t + t) * a.hq + h) * a.d;
+    } else {
+      src = a.k + b * a.kz + (int64_t)(h - a.hq) * a.kh + (int64_t)t * a.kt;
+      dst = a.ok + ((b * a.t + t) * a.hk + (h - a.hq)) * a.d;
+    }
+    const float c = (float)a.cs[b * a.cz + (int64_t)t * a.ct + d];
+    const float s = (float)a.sn[b * a.sz + (int64_t)t * a.st + d];
+    dst[d] = rope_one((float)src[d], (float)src[dr], c, s, sign);
   }
-  const float c = (float)a.cs[b * a.cz + (int64_t)t * a.ct + d];
-  const float s = (float)a.sn[b * a.sz + (int64_t)t * a.st + d];
-  dst[d] = rope_one((float)src[d], (float)src[dr], c, s, sign);
 }
 
 // ---- SiLU * up (reference :850-869) -----------------------------------------
@@ -352,20 +347,31 @@ int launch_rotary(const tilemix_rotary_params& p, hipStream_t stream) {
   a.hq = p.heads_q;
   a.hk = p.heads_k;
   a.d = p.head_dim;
-  a.bt = (int64_t)p.batch * p.tokens;
-  a.rows = a.bt * (p.heads_q + p.heads_k);
+  const int64_t heads = (int64_t)p.heads_q + p.heads_k;
+  a.rows = (int64_t)p.batch * p.tokens * heads;
   if (a.rows == 0) return TILEMIX_OK;
+  constexpr int64_t kMaxGroups = (1 << 24) - 1;  // of 256 threads: HIP takes less than 2^32 along x
+  // Whole tokens where that idles at most an eighth of the workgroup: its output then
+  // starts at a line's start more often (32768 tokens of 20 + 4 heads x 80 47.9 -> 44.8 us).
+  a.per_wg = std::max(1, 256 / std::max(1, p.head_dim / 16));
+  const int64_t whole = a.per_wg / heads * heads;
+  if (whole * 8 >= (int64_t)a.per_wg * 7) a.per_wg = (int)whole;
+  const int64_t groups = (a.rows - 1) / a.per_wg + 1;
   // 16-byte chunks need head_dim % 16 == 0 (so both halves are chunk aligned)
   // and every row start 16-byte aligned.
-  const bool vec = (p.head_dim % 16) == 0 && p.head_dim <= 16 * 256 && aligned16(p.q) && aligned16(p.k) && aligned16(p.cos) &&
-                   aligned16(p.sin) && aligned16(p.q_out) && aligned16(p.k_out) &&
+  const bool vec = (p.head_dim % 16) == 0 && p.head_dim <= 16 * 256 && a.rows <= INT32_MAX && groups <= kMaxGroups &&
+                   aligned16(p.q) && aligned16(p.k) && aligned16(p.cos) && aligned16(p.sin) && aligned16(p.q_out) &&
+                   aligned16(p.k_out) &&
                    ((a.qz | a.qh | a.qt | a.kz | a.kh | a.kt | a.cz | a.ct | a.sz | a.st) & 7) == 0;
   if (vec) {
-    const int64_t tokens = rot_tokens(p.head_dim / 16);
-    hipLaunchKernelGGL(rotary_kernel, dim3((unsigned)((a.bt + tokens - 1) / tokens)), dim3(256), 0, stream, a);
+    const int pairs = p.head_dim / 16;
+    a.by_pairs = make_fast_div(pairs);
+    a.by_heads = make_fast_div(p.heads_q + p.heads_k);
+    a.by_tokens = make_fast_div(p.tokens);
+    hipLaunchKernelGGL(rotary_kernel, dim3((unsigned)groups), dim3(256), 0, stream, a);
   } else {
-    const int64_t threads = a.rows * p.head_dim;
-    hipLaunchKernelGGL(rotary_kernel_scalar, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, a);
+    const int64_t all = std::min((a.rows * p.head_dim + 255) / 256, kMaxGroups);
+    hipLaunchKernelGGL(rotary_kernel_scalar, dim3((unsigned)all), dim3(256), 0, stream, a);
   }
   return check_launch("tilemix_rotary_f16");
 }
