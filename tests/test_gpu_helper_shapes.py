@@ -35,6 +35,20 @@ def test_rms_norm_row_stride_aligned_and_not(device):
         assert ok and frac <= 0.01, (width, frac)
 
 
+@pytest.mark.parametrize("cols,width", [(3072, 3076), (3072, 3075), (512, 516), (8192, 8196), (2056, 2060)])
+def test_rms_norm_aligned_rows_of_an_odd_stride(device, cols, width):
+    """Alignment is each row's own: the 16-byte aligned rows among unaligned ones have the bits of an aligned
+    tensor's (the order of the sum is the vector path's)."""
+    g = torch.Generator().manual_seed(cols + width)
+    base = torch.randn(256, width, generator=g).half().to(device)
+    w = (torch.randn(cols, generator=g) * 0.3 + 1.0).half().to(device)
+    rows = [r for r in range(256) if r * width % 8 == 0]
+    got, want = TL.rms_norm(base[:, :cols], w, 1e-5), TL.rms_norm(base[:, :cols].contiguous(), w, 1e-5)
+    assert torch.equal(got[rows], want[rows])
+    ok, frac = _within_ulps(got, PO.rms_norm(base[:, :cols].cpu(), w.cpu(), 1e-5), 2)
+    assert ok and frac <= 0.01, frac
+
+
 @pytest.mark.parametrize("b,hq,hk,t,d", [
     (1, 17, 1, 1, 16),      # one chunk pair per row, one head past the 16 slots
     (2, 33, 16, 5, 64),     # three passes over the head slots
