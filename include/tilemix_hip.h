@@ -37,7 +37,7 @@
 extern "C" {
 #endif
 
-#define TILEMIX_ABI_VERSION 3
+#define TILEMIX_ABI_VERSION 4
 
 enum tilemix_status {
     TILEMIX_OK = 0,

@@ -15,7 +15,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libtilemix_hip.so"
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 ROUTING_MIXED = 0
 ROUTING_FP16 = 1
@@ -141,6 +141,26 @@ def load_library(path: os.PathLike | str | None = None) -> ctypes.CDLL:
                 "(or __graft_entry__.build()); there is no CPU fallback"
             )
         lib = ctypes.CDLL(str(lib_path), mode=ctypes.RTLD_LOCAL)
+        # The version first: a library of another one may lack the symbols bound below.
+        missing = [name for name in EXPORTED_SYMBOLS if not hasattr(lib, name)]
+        if "tilemix_abi_version" in missing:
+            raise TileMixLibraryError(f"{lib_path} has no tilemix_abi_version; rebuild it")
+        lib.tilemix_abi_version.argtypes = []
+        lib.tilemix_abi_version.restype = ctypes.c_int
+        if lib.tilemix_abi_version() != ABI_VERSION:
+            raise TileMixLibraryError(
+                f"{lib_path}: ABI version {lib.tilemix_abi_version()} != {ABI_VERSION}; rebuild it"
+            )
+        if missing:
+            raise TileMixLibraryError(f"{lib_path} does not export {', '.join(missing)}; rebuild it")
+        lib.tilemix_params_size.argtypes = [ctypes.c_int]
+        lib.tilemix_params_size.restype = ctypes.c_int64
+        for which, struct in ((0, QuantParams), (1, AttnParams), (2, RmsNormParams), (3, RotaryParams)):
+            if lib.tilemix_params_size(which) != ctypes.sizeof(struct):
+                raise TileMixLibraryError(
+                    f"{lib_path}: {struct.__name__} size {lib.tilemix_params_size(which)} != "
+                    f"{ctypes.sizeof(struct)} (header and binding disagree); rebuild it"
+                )
         lib.tilemix_quant_per_block_int8.argtypes = [ctypes.POINTER(QuantParams), _vp]
         lib.tilemix_quant_per_block_int8.restype = ctypes.c_int
         lib.tilemix_quant_per_block_int8_many.argtypes = [ctypes.POINTER(QuantParams), _i32, _i32, _vp]
@@ -157,28 +177,26 @@ def load_library(path: os.PathLike | str | None = None) -> ctypes.CDLL:
         lib.tilemix_rotary_f16.restype = ctypes.c_int
         lib.tilemix_silu_mul_f16.argtypes = [_vp, _vp, _vp, _i64, _vp]
         lib.tilemix_silu_mul_f16.restype = ctypes.c_int
-        lib.tilemix_abi_version.argtypes = []
-        lib.tilemix_abi_version.restype = ctypes.c_int
-        lib.tilemix_params_size.argtypes = [ctypes.c_int]
-        lib.tilemix_params_size.restype = ctypes.c_int64
         lib.tilemix_last_error.argtypes = []
         lib.tilemix_last_error.restype = ctypes.c_char_p
-        if lib.tilemix_abi_version() != ABI_VERSION:
-            raise TileMixLibraryError(
-                f"{lib_path}: ABI version {lib.tilemix_abi_version()} != {ABI_VERSION}; rebuild it"
-            )
-        for which, struct in ((0, QuantParams), (1, AttnParams), (2, RmsNormParams), (3, RotaryParams)):
-            if lib.tilemix_params_size(which) != ctypes.sizeof(struct):
-                raise TileMixLibraryError(
-                    f"{lib_path}: {struct.__name__} size {lib.tilemix_params_size(which)} != "
-                    f"{ctypes.sizeof(struct)} (header and binding disagree); rebuild it"
-                )
         if path is None:
             _lib = lib
         return lib
 
 
 _host = None
+
+
+def _check_host(module, lib: ctypes.CDLL) -> None:
+    """``module`` passes the library its structs by layout and holds torch's C++ types: refuse one
+    that was compiled for another header or another torch."""
+    from .csrc.build import torch_id
+    built = module.built_for() if hasattr(module, "built_for") else None
+    now = (lib.tilemix_abi_version(), tuple(lib.tilemix_params_size(which) for which in range(4)), torch_id())
+    if built != now:
+        raise TileMixLibraryError(
+            f"tilemix_amd/_host.so was built for {built}, loaded are {now} (ABI version, struct sizes, torch): "
+            "rebuild it with `python -m tilemix_amd.csrc.build`")
 
 
 def host():
@@ -196,6 +214,7 @@ def host():
                 raise TileMixLibraryError(
                     f"tilemix_amd/_host.so cannot be loaded ({e}): build it with `python -m tilemix_amd.csrc.build` "
                     "(or __graft_entry__.build())") from e
+            _check_host(module, lib)
             module.bind(*(ctypes.cast(fn, _vp).value for fn in (
                 lib.tilemix_quant_per_block_int8_many, lib.tilemix_attn_fwd, lib.tilemix_attn_fwd_uniform,
                 lib.tilemix_rms_norm_f16, lib.tilemix_rotary_f16, lib.tilemix_silu_mul_f16)))

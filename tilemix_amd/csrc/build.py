@@ -70,13 +70,19 @@ def sources() -> list[Path]:
     return sorted(CSRC.glob("*.hip"))
 
 
+def torch_id() -> str:
+    """The torch that _host.so is compiled against: its C++ types have no stable layout."""
+    import torch
+    return f"{torch.__version__} {torch.version.git_version}"
+
+
 def _host_command(out: Path) -> list[str]:
     import torch
     root = Path(torch.__file__).resolve().parent
     includes = [root / "include", root / "include/torch/csrc/api/include", sysconfig.get_paths()["include"],
                 Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "include", INCLUDE]
     return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
-            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f'-DTILEMIX_TORCH="{torch_id()}"',
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
             *(arg for path in includes for arg in ("-isystem", str(path))), str(CSRC / "host.cpp"), "-o", str(out),
             f"-L{root / 'lib'}", f"-Wl,-rpath,{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]

@@ -61,6 +61,16 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Py_RETURN_NONE;
 }
 
+// built_for(): what this module was compiled against -- the ABI version and the sizes of the
+// parameter structs (as tilemix_params_size numbers them), and torch.  tilemix_amd/_native.py
+// compares them with what is loaded before it binds anything.
+PyObject* built_for(PyObject*, PyObject* const*, Py_ssize_t) {
+  return Py_BuildValue("(i(nnnn)s)", TILEMIX_ABI_VERSION, static_cast<Py_ssize_t>(sizeof(tilemix_quant_params)),
+                       static_cast<Py_ssize_t>(sizeof(tilemix_attn_params)),
+                       static_cast<Py_ssize_t>(sizeof(tilemix_rmsnorm_params)),
+                       static_cast<Py_ssize_t>(sizeof(tilemix_rotary_params)), TILEMIX_TORCH);
+}
+
 // ---- arguments ----------------------------------------------------------------
 
 // A torch.Tensor (no subclass) on a GPU whose storage the call may read directly.
@@ -567,7 +577,8 @@ PyMethodDef method(const char* name) {
   return PyMethodDef{name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(F)), METH_FASTCALL, nullptr};
 }
 
-PyMethodDef g_methods[] = {method<bind>("bind"),     method<packed>("packed"),     method<dense>("dense"),
+PyMethodDef g_methods[] = {method<built_for>("built_for"),
+                           method<bind>("bind"),     method<packed>("packed"),     method<dense>("dense"),
                            method<quantize>("quantize"),
                            method<rms_norm>("rms_norm"), method<rotary>("rotary"), method<silu_mul>("silu_mul"),
                            PyMethodDef{nullptr, nullptr, 0, nullptr}};
