@@ -79,6 +79,27 @@ def test_packed(device, both, mode, block_m, fp16_v, d):
         scalar_scales=block_m == 128, routing_mode=mode, int8_use_fp16_v=fp16_v)[0])
 
 
+@pytest.mark.parametrize("form", ["head_major", "fused_qkv", "one_head_expanded", "one_token"])
+@pytest.mark.parametrize("block_m", [64, 128])
+def test_packed_layouts(device, both, form, block_m):
+    """The output of a packed call has q's strides where q is dense (head-major q: head-major output)."""
+    g = torch.Generator(device=device).manual_seed(block_m)
+    n, hq, hk, d = 1 if form == "one_token" else 300, 4, 2, 64
+    q, k, v = (torch.randn(n, h, d, generator=g, device=device).half() for h in (hq, hk, hk))
+    if form in ("head_major", "one_token"):
+        q, k, v = (t.transpose(0, 1).contiguous().transpose(0, 1) for t in (q, k, v))
+    elif form == "fused_qkv":
+        q, k, v = torch.cat((q, k, v), dim=1).split([hq, hk, hk], dim=1)
+    else:
+        q = q[:, :1].expand(-1, hq, -1)
+    cu = torch.tensor([0, 1, n] if n > 1 else [0, n], dtype=torch.int32, device=device)
+    bits = _bitmask(hk, n, block_m, device)
+    out = both(lambda: tmx.tilemix_attention_with_quant(
+        q, k, v, cu, cu, n, n, bits, block_m=block_m, block_n=64, BLKQ=128, BLKK=64, causal=True,
+        scalar_scales=False, routing_mode="mixed", int8_use_fp16_v=True)[0])
+    assert out.stride() == torch.empty_like(q).stride()
+
+
 @pytest.mark.parametrize("form", ["token_major", "head_major_1", "fused_qkv", "wide_heads"])
 @pytest.mark.parametrize("d,length", [(64, 256), (128, 193), (80, 64), (112, 1)])
 def test_dense_layouts(device, both, form, d, length):

@@ -130,6 +130,7 @@ struct Call {
   int batch = 0, seqlen = 0;      // longest sequence (uniform: every one)
   int block_m = 0, block_n = 0, block_n_mask = 0, blkq = 0, blkk = 0;
   bool causal = false, fp16_v = false;
+  bool out_like_q = false;        // the output takes q's strides (else token-major)
   double sm_scale = 0;
   int mode = 0;
 };
@@ -175,6 +176,11 @@ at::Tensor launch(const Call& c) {
   const c10::DeviceGuard guard(device);
   void* const stream = c10::hip::getCurrentHIPStream(device.index()).stream();
   const auto options = at::TensorOptions().device(device);
+  at::Tensor out = c.out_like_q ? at::empty_like(*c.q.t)
+                                : at::empty({c.q.tokens, c.q.heads, d}, options.dtype(at::kHalf));
+  // The kernel writes four columns at a time.
+  if (out.stride(2) != 1 || out.stride(0) % 4 != 0 || out.stride(1) % 4 != 0 || !aligned(out.const_data_ptr(), 8))
+    return {};
 
   tilemix_attn_params p{};
   tilemix_quant_params quant[3]{};
@@ -246,7 +252,6 @@ at::Tensor launch(const Call& c) {
       p.stride_v8_head = d;
     }
   }
-  at::Tensor out = at::empty({c.q.tokens, c.q.heads, d}, options.dtype(at::kHalf));
   p.q = c.q.t->const_data_ptr();
   p.k = c.k.t->const_data_ptr();
   p.v = c.v.t->const_data_ptr();
@@ -260,8 +265,8 @@ at::Tensor launch(const Call& c) {
   p.stride_k_head = c.k.head_stride;
   p.stride_v_token = c.v.token_stride;
   p.stride_v_head = c.v.head_stride;
-  p.stride_o_token = c.q.heads * d;
-  p.stride_o_head = d;
+  p.stride_o_token = out.stride(0);
+  p.stride_o_head = out.stride(1);
   p.sm_scale = static_cast<float>(c.sm_scale);
   p.heads_q = static_cast<int32_t>(c.q.heads);
   p.heads_k = static_cast<int32_t>(c.k.heads);
@@ -324,6 +329,7 @@ PyObject* packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
   c.batch = static_cast<int>(cu_q->numel()) - 1;
   c.causal = causal != 0;
   c.fp16_v = fp16_v != 0;
+  c.out_like_q = true;
   at::Tensor out = launch(c);
   if (!out.defined()) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
