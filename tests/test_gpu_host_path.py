@@ -155,6 +155,10 @@ def test_not_served(device, both, form, monkeypatch):
                                                ("TILEMIX_BITMASK_ROUTING_MODE", " FP16", False),
                                                ("TILEMIX_SCORE_ONLY_PV", "0", True),
                                                ("TILEMIX_SCORE_ONLY_PV", "no", False),
+                                               ("TILEMIX_SCORE_ONLY_PV", "", True),
+                                               ("TILEMIX_BITMASK_ROUTING_MODE", "", True),
+                                               ("TILEMIX_FORCE_CONFIG", "", True),
+                                               ("TILEMIX_HIP_FUSED_Q_QUANT", "", False),
                                                ("TILEMIX_HIP_FUSED_Q_QUANT", "0", False)])
 def test_environment(device, both, monkeypatch, name, value, served):
     g = torch.Generator(device=device).manual_seed(6)

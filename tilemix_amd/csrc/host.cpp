@@ -146,7 +146,9 @@ int64_t up256(int64_t n) { return (n + 255) / 256 * 256; }
 // that this path serves.
 at::Tensor launch(const Call& c) {
   const int64_t d = c.q.dim, kv_rows = int64_t(c.seqlen) + 64;
-  if (g_lib.attn == nullptr || env_set("TILEMIX_FORCE_CONFIG") || env_set("TILEMIX_HIP_FUSED_Q_QUANT")) return {};
+  // (An empty TILEMIX_FORCE_CONFIG forces nothing; an empty TILEMIX_HIP_FUSED_Q_QUANT means off.)
+  if (g_lib.attn == nullptr || env_set("TILEMIX_FORCE_CONFIG") || std::getenv("TILEMIX_HIP_FUSED_Q_QUANT") != nullptr)
+    return {};
   if (c.k.tokens != c.v.tokens || c.k.heads != c.v.heads || c.k.dim != d || c.v.dim != d || d <= 0 || d > 128 ||
       d % 16 != 0)
     return {};
