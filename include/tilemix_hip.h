@@ -251,7 +251,8 @@ int tilemix_rotary_f16(const tilemix_rotary_params* p, void* stream);
  * SiLU(gate) * up.  Replaces the _silu_mul Triton kernel and silu_mul
  * (models/tilemix_llama.py:850-869):
  *   out[i] = fp16( fp32( fp16( g / (1 + exp(-g)) ) ) * fp32(up[i]) ),  g = fp32(gate[i])
- * with a correctly rounded fp32 quotient.  gate, up and out are contiguous, n elements.
+ * whose quotient, rounded to fp16, is that of an IEEE fp32 division.  gate, up and
+ * out are contiguous, n elements.
  */
 int tilemix_silu_mul_f16(const void* gate, const void* up, void* out, int64_t n, void* stream);
 

@@ -83,3 +83,13 @@ def test_silu_mul_every_gate(device, up):
     assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)]) and torch.isfinite(got[finite]).all()
     ok, frac = _within_ulps(got[finite], want[finite], 1)
     assert ok and frac <= 1e-3, frac
+
+
+def test_silu_mul_smallest_gates(device):
+    """The gates up to 2^-20, exactly: there exp(-g) and the denominators are the nearest fp32 values, and a
+    quotient one ulp off (the denominator 2 - 2^-23) would show in no other gate."""
+    gate = torch.arange(0, 17, dtype=torch.int16).view(torch.float16)
+    gate = torch.cat((gate, -gate))
+    ones = torch.ones_like(gate)
+    got, want = TL.silu_mul(gate.to(device), ones.to(device)).cpu(), PO.silu_mul(gate, ones)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))

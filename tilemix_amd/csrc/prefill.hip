@@ -220,13 +220,15 @@ __global__ void __launch_bounds__(256) rotary_kernel_scalar(const RotaryArgs a) 
 }
 
 // ---- SiLU * up (reference :850-869) -----------------------------------------
-// g / den correctly rounded (den >= 1): a Newton step on the hardware reciprocal,
-// Markstein's correction of the quotient, and the fix-up instruction for
-// infinities and NaNs.  A quotient too small for its remainder to be exact lies
-// far below half of fp16's smallest value and becomes 0 either way; a denominator
-// of infinity (exp(-g) overflows) is such a case.  The full IEEE division adds
-// scaling steps for ranges that do not occur here; all 65536 gate values give the
-// same bits.  2048 x 8192: 19.5 -> 18.4 us; 32768 x 8192 is HBM-bound either way
+// g / den (den >= 1): a Newton step on the hardware reciprocal, Markstein's
+// correction of the quotient, and the fix-up instruction for infinities and NaNs.
+// Correctly rounded, but for den = 2 - 2^-23 with a reciprocal that is not the nearest
+// (one ulp then, which no fp16 result shows as exp is exact enough there).  A
+// quotient too small for its remainder to be exact lies far below half of fp16's
+// smallest value and becomes 0 either way; a denominator of infinity (exp(-g)
+// overflows) is such a case.  The full IEEE division adds
+// scaling steps for ranges that do not occur here; every gate gives the same fp16
+// value, whichever reciprocal within one ulp the instruction returns.  2048 x 8192: 19.5 -> 18.4 us; 32768 x 8192 is HBM-bound either way
 // (276 -> 273 us, 5.9 TB/s).
 __device__ __forceinline__ float silu_div(float g, float den) {
   float r = __builtin_amdgcn_rcpf(den);
