@@ -1,6 +1,7 @@
-// Host-side dump of the attention kernels' workgroup -> work-item mapping
-// (work_item in attn_common.h) for tests/test_work_item.py:
-//   work_item_dump groups m_blocks group ilv  ->  one line per workgroup: "bid item"
+// Host-side dump of the attention kernels' position -> work-item mapping
+// (work_position in attn_common.h, before spread_workgroup orders the positions) for
+// tests/test_work_item.py:
+//   work_item_dump groups m_blocks group ilv  ->  one line per position: "position item"
 //   work_item_dump --ilv max_seqlen_k head_dim  ->  interleave_groups
 #include <cstdio>
 #include <cstdlib>
@@ -18,7 +19,10 @@ int main(int argc, char** argv) {
   const long ipg = m_blocks * group;
   const long total = groups * ipg;
   const long grid = 8 * tmx::work_items_per_xcd(groups, ipg);
-  for (long bid = 0; bid < grid; ++bid)
-    printf("%ld %d\n", bid, tmx::work_item((int)bid, (int)total, (int)ipg, ilv));
+  const tmx::WorkMap w = tmx::make_work_map((int)total, (int)ipg, ilv, 1, 1);
+  for (long p = 0; p < grid; ++p) {
+    int grp, item;
+    printf("%ld %ld\n", p, tmx::work_position(w, (int)p, grp, item) ? grp * ipg + item : -1L);
+  }
   return 0;
 }

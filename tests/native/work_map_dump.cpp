@@ -1,6 +1,6 @@
 // Host-side dump of the attention kernels' launch order (spread_workgroup, then
 // work_position, attn_common.h) and of fast_div, for tests/test_work_map.py:
-//   work_map_dump groups m_blocks group ilv [workgroups per CU]  ->  one line per workgroup: "bid group item" (-1 -1: none)
+//   work_map_dump groups m_blocks group ilv [workgroups per CU [causal]]  ->  one line per workgroup: "bid group item" (-1 -1: none)
 //   work_map_dump --div                      ->  the number of wrong quotients over edges and a sweep
 #include <cstdio>
 #include <cstdlib>
@@ -25,10 +25,11 @@ int main(int argc, char** argv) {
     printf("%ld\n", wrong);
     return 0;
   }
-  if (argc != 5 && argc != 6) return 2;
+  if (argc < 5 || argc > 7) return 2;
   const int groups = atoi(argv[1]), m_blocks = atoi(argv[2]), group = atoi(argv[3]), ilv = atoi(argv[4]);
   const int ipg = m_blocks * group;
-  const tmx::WorkMap w = tmx::make_work_map(groups * ipg, ipg, ilv, group, 1, true, argc == 6 ? atoi(argv[5]) : 2);
+  const tmx::WorkMap w = tmx::make_work_map(groups * ipg, ipg, ilv, group, 1, argc < 7 || atoi(argv[6]) != 0,
+                                            argc > 5 ? atoi(argv[5]) : 2);
   for (int bid = 0; bid < 8 * w.per_xcd; ++bid) {
     int grp = -1, item = -1;
     if (!tmx::work_position(w, tmx::spread_workgroup(w, bid), grp, item)) grp = item = -1;

@@ -1,5 +1,6 @@
-"""The workgroup -> work-item mapping of the attention kernels (work_item in
-tilemix_amd/csrc/attn_common.h), compiled for the host with hipcc and checked
+"""The position -> work-item mapping of the attention kernels (work_position in
+tilemix_amd/csrc/attn_common.h; the order in which workgroups take the positions is
+test_work_map.py's), compiled for the host with hipcc and checked
 on the CPU: every item is processed exactly once, a group of a whole round
 stays on one XCD, the XCD's groups run `ilv` at a time interleaved item by
 item, each group's query blocks longest first; and the interleave chosen per

@@ -93,3 +93,32 @@ def test_three_workgroups_per_cu(dump_bin, groups, m_blocks, group):
         assert all(at[j] == j for j in range(32))
         assert all(at[j + 32] == 63 - j for j in range(32))
         assert all(at[j] == j for j in range(64, n))
+
+
+@pytest.mark.parametrize("per_cu", [2, 3])
+@pytest.mark.parametrize("groups,m_blocks,group", [(4, 16, 7), (1, 33, 8), (7, 13, 4), (4, 22, 7), (5, 31, 4), (1, 96, 8),
+                                                   (2, 65, 4)])
+def test_shared_cus_with_fewer_than_8_groups(dump_bin, groups, m_blocks, group, per_cu):
+    """33 to 96 workgroups per XCD of launches whose groups are dealt over all XCDs: every item once; with
+    two per CU and the groups interleaved all at once, the longest items are alone."""
+    rows = [tuple(map(int, ln.split())) for ln in _run(dump_bin, groups, m_blocks, group, 4, per_cu).splitlines()]
+    n = len(rows) // 8
+    assert 32 < n <= 96
+    assert sorted((g, i) for _, g, i in rows if g >= 0) == [(g, i) for g in range(groups)
+                                                            for i in range(m_blocks * group)]
+    if n <= 64 and groups <= 4:
+        for x in range(8):
+            item = [rows[8 * j + x][2] for j in range(n)]
+            alone = [item[j] for j in range(n - 32, 32) if item[j] >= 0]
+            paired = [item[j] for j in (*range(n - 32), *range(32, n)) if item[j] >= 0]
+            assert not alone or max(alone) <= min(paired)
+
+
+@pytest.mark.parametrize("per_cu", [2, 3])
+@pytest.mark.parametrize("groups,m_blocks,group", [(8, 11, 3), (8, 24, 4), (4, 16, 7), (64, 15, 4), (3, 40, 1)])
+def test_without_the_causal_limit(dump_bin, groups, m_blocks, group, per_cu):
+    """Items of equal length: the rotated order, whatever number of workgroups a CU holds."""
+    rows = _run(dump_bin, groups, m_blocks, group, 4, per_cu, 0)
+    assert rows == _run(dump_bin, groups, m_blocks, group, 4, 1, 1)  # one workgroup per CU: nothing shared
+    done = [tuple(map(int, ln.split()[1:])) for ln in rows.splitlines()]
+    assert sorted(p for p in done if p[0] >= 0) == [(g, i) for g in range(groups) for i in range(m_blocks * group)]

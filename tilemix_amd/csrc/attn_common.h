@@ -10,8 +10,8 @@ namespace tmx {
 
 constexpr int kBN = 64;  // keys per compute tile (block_n)
 
-// n / d for 0 <= n < 2^31 by a multiplication: with 2^shift the smallest power of
-// two >= d, q = (n + hi32(n * mul)) >> shift (three scalar instructions where a
+// n / d for 0 <= n < 2^31 by a multiplication (Granlund and Montgomery's division by
+// an invariant integer): with 2^shift the smallest power of two >= d, q = (n + hi32(n * mul)) >> shift (three scalar instructions where a
 // division by a kernel argument takes about thirty, in series).
 struct FastDiv {
   uint32_t mul;
@@ -141,12 +141,6 @@ __host__ __device__ __forceinline__ bool work_position(const WorkMap& w, int bid
   item = fast_div(p, by_kc);
   grp = 8 * w.gpx + c * w.ilv + p - item * by_kc.d;
   return n < w.tail * w.ipg;
-}
-// The same as an item number, or -1 (host: the mapping's test).
-inline int work_item(int bid, int total_items, int ipg, int ilv) {
-  const WorkMap w = make_work_map(total_items, ipg, ilv, 1, 1);
-  int grp, item;
-  return work_position(w, bid, grp, item) ? grp * ipg + item : -1;
 }
 
 struct AttnKArgs {
