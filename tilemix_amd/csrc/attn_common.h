@@ -99,13 +99,22 @@ inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int h
 // with shortest.  Against longest first throughout (us, K quantisation included): 24/8
 // heads 1 x 1537 38.7 -> 37.1, 1 x 2048 51.0 -> 48.0 (fp16 mode 46.2 -> 42.9), 3 x 700
 // 28.7 -> 27.1; 28/4 heads 1 x 1537 40.6 -> 38.6, 1 x 2200 58.2 -> 55.4.
+// Packed prompts of different lengths, whose positions are not in order of length,
+// gain as well, against the rotation (us, mixed mode; the other modes and int8 V 1% more
+// to 20% less): 24/8 heads 4 of 60 .. 512 24.2 -> 22.0, 2 of 200 .. 1024 30.8 ->
+// 28.9; 32/8 heads 4 of 100 .. 512 23.8 -> 22.5; 28/4 heads 2 of 400 .. 1000 34.6 -> 31.9;
+// 4/1 heads 6 of 300 .. 2200 64.8 -> 54.3; 24/8 heads 8 of 40 .. 256 20.1 either way.
 //
 // At head_dim <= 64 a CU holds three workgroups, and with 65 to 96 per XCD all start
 // at once as well, by threes (j, j + 32, j + 64).  The longest 32 keep their places,
 // the next 32 run in the opposite order, the rest follows.  Against the rotation (us,
 // causal, head_dim 64, 32/8 heads; the repeats differ by up to 0.6): fp16 mode 1 x 2200
 // 39.4 -> 37.2, 1 x 2600 47.1 -> 42.4, 1 x 3072 59.5 -> 54.2; mixed mode 1 x 2600
-// 56.2 -> 55.8, 1 x 3072 69.3 -> 69.5; 14/2 heads 1 x 5000 100.0 -> 98.1.
+// 56.2 -> 55.8, 1 x 3072 69.3 -> 69.5; 14/2 heads 1 x 5000 100.0 -> 98.1.  int8 mode 1 x
+// 2600 53.1 -> 48.5, 1 x 3072 66.3 -> 60.3; with int8 V 61.6 -> 60.5 and 76.8 -> 73.3, mixed
+// mode with int8 V within 1%.  Packed prompts, mixed / fp16 / int8 mode: 300, 500, 200
+// and 768 tokens 24.4 -> 23.6 / 17.4 -> 14.6 / 23.4 -> 20.4, 700 and 1536 38.2 -> 37.9 /
+// 29.4 -> 27.5 / 36.2 -> 33.8.
 __host__ __device__ __forceinline__ int spread_workgroup(const WorkMap& w, int bid) {
   const int x = bid & 7, j = bid >> 3;
   const int base = j < w.full_j ? 0 : w.full_j, n = j < w.full_j ? w.full_j : w.per_xcd - w.full_j;
