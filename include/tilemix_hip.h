@@ -123,7 +123,8 @@ int tilemix_quant_per_block_int8_many(const tilemix_quant_params* p, int32_t cou
  * Supported by this build: block_m in {64, 128, 256, 512}; block_n in {64, 128, 256};
  * block_n_mask a multiple of block_n with ceil(max_seqlen_k/block_n_mask) <= 64;
  * head_dim a multiple of 16, <= 128 (the Python layer zero-pads other widths);
- * blkk a positive multiple of 4; fp16 data; (max_seqlen_k + 64) times the
+ * blkk a positive multiple of 4; fp16 data; token strides of at least head_dim
+ * (reads are bounded by length times stride); (max_seqlen_k + 64) times the
  * largest K/V token stride in bytes below 2 GiB and 128 Q token strides below
  * 2 GiB (tiles are read through 32-bit buffer offsets; the Python layer passes
  * a head-major copy of a stream whose strides exceed it, as the reference

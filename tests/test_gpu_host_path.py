@@ -123,6 +123,38 @@ def test_dense_layouts(device, both, form, d, length):
     assert out.shape == (b, hq, length, d)
 
 
+@pytest.mark.parametrize("form", ["expanded", "overlapping", "one_token"])
+@pytest.mark.parametrize("operand", [0, 1, 2])
+def test_tokens_closer_than_their_rows(device, form, operand):
+    """One sequence whose tokens repeat, overlap, or (one token) have a stride that says nothing: the result of
+    the dense tensors, through both entry points."""
+    g = torch.Generator(device=device).manual_seed(operand)
+    n, h, d = 1 if form == "one_token" else 150, 2, 64
+    x = [torch.randn(1, n, h, d, generator=g, device=device).half().transpose(1, 2) for _ in range(3)]
+    if form == "expanded":
+        x[operand] = x[operand][:, :, :1].expand(-1, -1, n, -1)
+    elif form == "overlapping":
+        base = torch.randn(h, 8 * n + d, generator=g, device=device).half()
+        x[operand] = base.as_strided((1, h, n, d), (0, 8 * n + d, 8, 1))
+    else:
+        x[operand] = x[operand].as_strided((1, h, 1, d), (0, d, 0, 1))
+    dense = [t.clone(memory_format=torch.contiguous_format) for t in x]
+    bits = _bitmask(h, n, 64, device)
+    cu = torch.tensor([0, n], dtype=torch.int32, device=device)
+
+    def call(q, k, v):
+        return tilemix_varlen_attention(q, k, v, 64, 64, causal=True, scale=0.125, precision_map_all=bits,
+                                        candidates=[], flat_lengths=[])
+
+    def packed(*qkv):
+        return tmx.tilemix_attention_with_quant(
+            *(t[0].transpose(0, 1) for t in qkv), cu, cu, n, n, bits, block_m=64, block_n=64, causal=True,
+            scalar_scales=False, routing_mode="mixed", int8_use_fp16_v=True)[0]
+
+    assert torch.equal(call(*x), call(*dense))
+    assert torch.equal(packed(*x), packed(*dense))
+
+
 @pytest.mark.parametrize("form", ["head_major", "misaligned", "head_dim_72", "map_on_cpu", "int64_cu", "bias", "forced"])
 def test_not_served(device, both, form, monkeypatch):
     """Calls that need a copy, a conversion, padding or a switch go through the Python path."""

@@ -66,3 +66,20 @@ def test_quantisation_block_limit(lib):
     p[0].heads, p[0].head_dim, p[0].blk_tokens, p[0].batch, p[0].max_seqlen = 1, 8, 1, 1, 1 << 24
     assert lib.tilemix_quant_per_block_int8_many(p, 1, 0, None) == 1
     assert b"at most 16777215 blocks" in lib.tilemix_last_error()
+
+
+def test_attention_token_stride(lib):
+    """Tokens closer than their rows are long are refused (a sequence's reads are bounded by its length
+    times the token stride, so the last rows would read zeros)."""
+    p = _native.AttnParams()
+    for f in ("q", "k", "v", "out", "precision_bitmask", "cu_seqlens_q", "cu_seqlens_k"):
+        setattr(p, f, ctypes.c_void_p(1 << 12))
+    p.heads_q = p.heads_k = p.batch = 1
+    p.head_dim, p.max_seqlen_q, p.max_seqlen_k = 64, 128, 128
+    p.block_m, p.block_n, p.block_n_mask, p.blkq, p.blkk, p.routing_mode = 128, 64, 64, 128, 64, 1
+    strides = ("stride_q_token", "stride_k_token", "stride_v_token")
+    for short in strides:
+        for f in strides:
+            setattr(p, f, 56 if f == short else 64)
+        assert lib.tilemix_attn_fwd(ctypes.byref(p), None) == 1
+        assert b"token strides must be at least head_dim" in lib.tilemix_last_error()

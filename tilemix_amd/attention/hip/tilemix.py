@@ -238,10 +238,13 @@ def _pad_head_dim(t: Optional[torch.Tensor], width: int) -> Optional[torch.Tenso
 
 
 def _inner_contiguous(t: torch.Tensor, align: int) -> torch.Tensor:
-    """The kernel reads 16-byte vectors along the head dim: unit dim stride and
-    vector-aligned token/head strides; otherwise take a dense copy."""
-    if t.stride(2) != 1 or t.stride(0) % align or t.stride(1) % align or t.data_ptr() % 16:
-        return t.contiguous()
+    """The kernel reads 16-byte vectors along the head dim and bounds a sequence's reads by its
+    length times the token stride: unit dim stride, vector-aligned token/head strides and tokens
+    no closer than their rows are long (an expanded or overlapping token dimension); otherwise
+    take a dense copy (``contiguous()`` would keep the strides of dimensions of size one)."""
+    if (t.stride(2) != 1 or t.stride(0) % align or t.stride(1) % align or t.stride(0) < t.shape[2]
+            or t.data_ptr() % 16):
+        return t.clone(memory_format=torch.contiguous_format)
     return t
 
 

@@ -154,6 +154,14 @@ int launch_attn(const tilemix_attn_params& p, int uniform_seqlen, int32_t* dump_
     return TILEMIX_E_INVALID;
   }
 
+  // A sequence's reads are bounded by its length times the token stride.
+  if (std::min(std::min(p.stride_q_token, p.stride_k_token), p.stride_v_token) < p.head_dim ||
+      (need_int8 && ((!p.q_quant_in_kernel && p.stride_q8_token < p.head_dim) || p.stride_k8_token < p.head_dim ||
+                     (int8v && p.stride_v8_token < p.head_dim)))) {
+    set_error("%s: token strides must be at least head_dim (%d)", fn, p.head_dim);
+    return TILEMIX_E_INVALID;
+  }
+
   const int m_blocks = (p.max_seqlen_q + wg_rows - 1) / wg_rows;
   const int64_t total = (int64_t)m_blocks * p.heads_q * p.batch;
   if (total == 0) return TILEMIX_OK;

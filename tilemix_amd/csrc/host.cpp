@@ -115,10 +115,11 @@ struct Operand {
   const at::Tensor* t = nullptr;
   int64_t tokens = 0, heads = 0, dim = 0, token_stride = 0, head_stride = 0;
 
-  // Read as it lies: 16-byte vectors, and `rows` token strides below 2 GiB.
+  // Read as it lies: 16-byte vectors, `rows` token strides below 2 GiB, and tokens no closer than
+  // their rows are long (the kernels bound a sequence's reads by its length times the stride).
   bool direct(int64_t rows) const {
-    return token_stride % 8 == 0 && head_stride % 8 == 0 && aligned(t->const_data_ptr(), 16) &&
-           rows * token_stride * 2 < kSpan;
+    return token_stride % 8 == 0 && head_stride % 8 == 0 && token_stride >= dim &&
+           aligned(t->const_data_ptr(), 16) && rows * token_stride * 2 < kSpan;
   }
 };
 
