@@ -29,9 +29,11 @@
 // their chain of scalar loads and divisions before the first row (or the exit).  Divisors
 // come as multipliers from the host, a launch of one tensor reads its arguments at
 // once, the maximum takes one barrier.  With the divisions, a tensor chosen after a
-// load and two barriers (us): 8192 tokens x 8 heads x 128 in blocks of 1 101 -> 63, of 4
-// 28.4 -> 18.7, of 64 6.6 -> 5.9; 200 prompts of 5 tokens and one of 8000, blocks of 64
-// 161 -> 49.
+// load and two barriers (us): 8192 tokens x 8 heads x 128 in blocks of 1 101 -> 60, of 4
+// 28.0 -> 17.7, of 64 6.5 -> 5.8; 200 prompts of 5 tokens and one of 8000, blocks of 64
+// 161 -> 48.  The loads of a block's rows are unconditional (a row past the block is its
+// first one again), so that they go out together: as conditional ones the first was
+// waited for alone, and K and V of 8192 tokens x 8 heads x 128 took 11.4 us instead of 10.5.
 #include "attn_common.h"
 
 #include <algorithm>
@@ -104,7 +106,7 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int id = blockIdx.x, b = blockIdx.y;
   const int tensor = MANY ? (id >= args.first[1]) + (id >= args.first[2]) : 0;
-  const QuantTensor& a = args.t[tensor];
+  const QuantTensor a = args.t[tensor];  // a copy: by reference each argument's load waits for its use
   const int uni = args.uni;
   const int t = MANY ? id - args.first[tensor] : id;
   const int row = fast_div(t, a.by_heads), heads = a.by_heads.d, h = t - row * heads;
@@ -123,14 +125,22 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
   // that stores the scale adds them behind the maximum's barrier.  The sum is a chain
   // of loads, so all four waves share it and each keeps four loads in flight: by one
   // wave alone, a load at a time, 4096 sequences of 16 tokens x 8 heads x 128 take 126 us
-  // instead of 81, 8192 of 4 tokens 367 instead of 187.
+  // instead of 73, 8192 of 4 tokens 367 instead of 170.
   auto scale_rows = [&](int n) { return n > 0 ? fast_div(n - 1, a.by_blk) + 1 : 0; };
   auto sum_scale_rows = [&]() {
     if (uni > 0) return;
     int part = 0;
     if (b > wave * 64) {
-#pragma unroll 4
-      for (int bb = tid; bb < b; bb += kQuantThreads) part += scale_rows(a.cu[bb + 1] - a.cu[bb]);
+      for (int b0 = tid; b0 < b; b0 += 4 * kQuantThreads) {
+        int len4[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int bb = min(b0 + i * kQuantThreads, b);
+          len4[i] = a.cu[bb + 1] - a.cu[bb];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part += b0 + i * kQuantThreads < b ? scale_rows(len4[i]) : 0;
+      }
       part = wave_sum_i(part);
     }
     if (lane == 0) red_rows[wave] = part;
@@ -161,7 +171,8 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
   const int r0 = fast_div(tid, a.by_chunks), col = (tid - r0 * a.by_chunks.d) << 3;
   const bool used = r0 < rpi;  // the chunks per row need not divide the workgroup
   const int64_t tok0 = (int64_t)start + (int64_t)blk * blk_tokens;
-  const f16* in = a.in + (tok0 + r0) * a.si_t + (int64_t)h * a.si_h + col;
+  const f16* in_row0 = a.in + tok0 * a.si_t + (int64_t)h * a.si_h + col;
+  const f16* in = in_row0 + (int64_t)r0 * a.si_t;
   int8_t* out = a.out + (tok0 + r0) * a.so_t + (int64_t)h * a.so_h + col;
   const int64_t in_step = (int64_t)rpi * a.si_t, out_step = (int64_t)rpi * a.so_t;
 
@@ -235,10 +246,8 @@ __global__ void __launch_bounds__(kQuantThreads) quant_per_block_int8_kernel(con
     u32x4 xs[kN];
     uint32_t m2 = 0;
 #pragma unroll
-    for (int i = 0; i < kN; ++i) {
-      xs[i] = (u32x4){};
-      if (used && r0 + i * rpi < rows) xs[i] = *reinterpret_cast<const u32x4*>(in + i * in_step);
-    }
+    for (int i = 0; i < kN; ++i)  // past the block: its first row once more, which leaves the maximum as it is
+      xs[i] = *reinterpret_cast<const u32x4*>(used && r0 + i * rpi < rows ? in + i * in_step : in_row0);
     sum_scale_rows();
 #pragma unroll
     for (int i = 0; i < kN; ++i) m2 = magnitudes(xs[i], m2);
