@@ -8,9 +8,9 @@
 // always did; so does a call whose launch fails.  The checks below are those of
 // the Python path plus the conditions under which it would copy.
 //
-// Why: a 256-token call has ~17 us of GPU work, and the Python path (attribute
+// Why: a 256-token call has ~12 us of GPU work, and the Python path (attribute
 // reads, ~60 ctypes fields, six allocations, two device contexts) took ~70 us of
-// host time per call; this one takes ~8 us.
+// host time per call; this one takes ~9 us.
 //
 // The GPU library stays free of torch: its entry points are bound by address
 // (bind(), from the ctypes handle of tilemix_amd/_native.py).
