@@ -35,7 +35,8 @@ def test_rms_norm_row_stride_aligned_and_not(device):
         assert ok and frac <= 0.01, (width, frac)
 
 
-@pytest.mark.parametrize("cols,width", [(3072, 3076), (3072, 3075), (512, 516), (8192, 8196), (2056, 2060)])
+@pytest.mark.parametrize("cols,width", [(3072, 3076), (3072, 3075), (512, 516), (8192, 8196), (2056, 2060),
+                                        (4096, 4100), (4104, 4108), (6400, 6402), (8184, 8196)])
 def test_rms_norm_aligned_rows_of_an_odd_stride(device, cols, width):
     """Alignment is each row's own: the 16-byte aligned rows among unaligned ones have the bits of an aligned
     tensor's (the order of the sum is the vector path's)."""

@@ -57,6 +57,8 @@ __device__ __forceinline__ float add_square(uint32_t h2, float acc, bool high) {
 // (us): 32768 x 3072 88 -> 78 (5.2 TB/s, a large copy's rate), 8192 x 2048 15.6 -> 12.8,
 // 2048 x 3072 7.8 -> 7.0, 4096 x 8192 23.5 -> 22.9.
 constexpr int kNormWaves = 4;
+constexpr int kNormChunks = 16;  // chunks per lane of the longest rows that are read in chunks
+constexpr int kNormStep = 4;     // chunks in flight per lane where a row is read twice
 
 struct NormArgs {
   const f16* x;
@@ -78,11 +80,14 @@ __device__ __forceinline__ f16 norm_one(float x, float rs, f16 w) {
   return (f16)((float)w * (float)hn);        // fp16(fp32(w) * fp32(hn))
 }
 
-// NCH: 8-element chunks a lane holds; 0 = rows longer than 16 chunks a lane.  Those,
-// and the rows that are not 16-byte aligned, go element by element.  ALIGNED: every
+// NCH: 8-element chunks a lane holds; 0: none.  Rows longer than 16 chunks a lane, and
+// the rows that are not 16-byte aligned, go element by element.  ALIGNED: every
 // row is (asking each row costs 64 rows of 3072 3.54 instead of 3.46 us).  Of rows 3076
 // elements apart every other one is aligned: 2048 of them 18.3 us element by element,
-// 16.3 so; 16384 71.7 and 63.8.
+// 16.3 so; 16384 71.7 and 63.8.  With more than 8 chunks a lane the registers that
+// hold an aligned row would cost the other rows the waves that hide their loads (16384
+// rows, us: 6402 wide 329 -> 199, 7753 396 -> 261, 5120 of 5124 186 -> 130), so NCH = 0 reads
+// its aligned rows twice; up to 8 chunks that gains nothing (4096 of 4100 86 -> 91).
 template <int NCH, bool ALIGNED>
 __global__ void __launch_bounds__(kNormWaves * 64) rmsnorm_kernel(const NormArgs a) {
   const int lane = threadIdx.x & 63;
@@ -93,9 +98,22 @@ __global__ void __launch_bounds__(kNormWaves * 64) rmsnorm_kernel(const NormArgs
   const int chunks = a.cols >> 3;          // full 8-element chunks
   const int tail0 = chunks << 3;           // first element of the ragged tail
   float ss = 0.0f;
-  const bool vec = NCH > 0 && (ALIGNED || ((reinterpret_cast<uintptr_t>(xr) | reinterpret_cast<uintptr_t>(orow) |
-                                            reinterpret_cast<uintptr_t>(a.w)) & 15) == 0);
-  if (vec) {
+  auto aligned_row = [&]() {
+    return ((reinterpret_cast<uintptr_t>(xr) | reinterpret_cast<uintptr_t>(orow) | reinterpret_cast<uintptr_t>(a.w)) &
+            15) == 0;
+  };
+  auto factor = [&]() {
+    const float var = wave_sum(ss) * a.inv_cols;
+    return 1.0f / sqrtf(var + a.eps);
+  };
+  auto store_chunk = [&](int c, const u32x4& x, float rs) {
+    const f16x8 wv = *reinterpret_cast<const f16x8*>(a.w + c * 8);
+    f16x8 hn;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) hn[e] = (f16)mul_half(x[e >> 1], rs, e & 1);
+    *reinterpret_cast<f16x8*>(orow + c * 8) = wv * hn;
+  };
+  if (NCH > 0 && (ALIGNED || aligned_row())) {
     u32x4 xv[NCH > 0 ? NCH : 1];
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
@@ -108,24 +126,43 @@ __global__ void __launch_bounds__(kNormWaves * 64) rmsnorm_kernel(const NormArgs
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss = add_square(xv[i][e >> 1], ss, e & 1);
     for (int c = tail0 + lane; c < a.cols; c += 64) ss += (float)xr[c] * (float)xr[c];
-    const float var = wave_sum(ss) * a.inv_cols;
-    const float rs = 1.0f / sqrtf(var + a.eps);
+    const float rs = factor();
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int c = i * 64 + lane;
-      if (c < chunks) {
-        const f16x8 wv = *reinterpret_cast<const f16x8*>(a.w + c * 8);
-        f16x8 hn;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) hn[e] = (f16)mul_half(xv[i][e >> 1], rs, e & 1);
-        *reinterpret_cast<f16x8*>(orow + c * 8) = wv * hn;
-      }
+      if (c < chunks) store_chunk(c, xv[i], rs);
     }
+    for (int c = tail0 + lane; c < a.cols; c += 64) orow[c] = norm_one((float)xr[c], rs, a.w[c]);
+  } else if (NCH == 0 && chunks <= kNormChunks * 64 && aligned_row()) {
+    // the same sums, kNormStep chunks at a time
+    auto each_step = [&](auto&& use) {
+      for (int c0 = lane; c0 < chunks; c0 += 64 * kNormStep) {
+        u32x4 xv[kNormStep];
+#pragma unroll
+        for (int i = 0; i < kNormStep; ++i) {
+          xv[i] = (u32x4){};
+          if (c0 + i * 64 < chunks) xv[i] = *reinterpret_cast<const u32x4*>(xr + (c0 + i * 64) * 8);
+        }
+        use(c0, xv);
+      }
+    };
+    each_step([&](int, const u32x4(&xv)[kNormStep]) {
+#pragma unroll
+      for (int i = 0; i < kNormStep; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = add_square(xv[i][e >> 1], ss, e & 1);
+    });
+    for (int c = tail0 + lane; c < a.cols; c += 64) ss += (float)xr[c] * (float)xr[c];
+    const float rs = factor();
+    each_step([&](int c0, const u32x4(&xv)[kNormStep]) {
+#pragma unroll
+      for (int i = 0; i < kNormStep; ++i)
+        if (c0 + i * 64 < chunks) store_chunk(c0 + i * 64, xv[i], rs);
+    });
     for (int c = tail0 + lane; c < a.cols; c += 64) orow[c] = norm_one((float)xr[c], rs, a.w[c]);
   } else {
     for (int c = lane; c < a.cols; c += 64) ss += (float)xr[c] * (float)xr[c];
-    const float var = wave_sum(ss) * a.inv_cols;
-    const float rs = 1.0f / sqrtf(var + a.eps);
+    const float rs = factor();
     for (int c = lane; c < a.cols; c += 64) orow[c] = norm_one((float)xr[c], rs, a.w[c]);
   }
 }
@@ -278,7 +315,10 @@ template <bool ALIGNED>
 static void launch_norm(const NormArgs& a, hipStream_t stream) {
   const int lane_chunks = (a.cols / 8 + 63) / 64;  // per lane
   const dim3 grid((unsigned)((a.rows + kNormWaves - 1) / kNormWaves)), block(kNormWaves * 64);
-  switch (lane_chunks > 16 ? 0 : lane_chunks > 8 ? 16 : lane_chunks > 6 ? 8 : (lane_chunks + 1) / 2 * 2) {
+  switch (lane_chunks > (ALIGNED ? kNormChunks : 8) ? 0
+          : lane_chunks > 8                         ? kNormChunks
+          : lane_chunks > 6                         ? 8
+                                                    : (lane_chunks + 1) / 2 * 2) {
     case 2:
       hipLaunchKernelGGL((rmsnorm_kernel<2, ALIGNED>), grid, block, 0, stream, a);
       break;
@@ -291,8 +331,8 @@ static void launch_norm(const NormArgs& a, hipStream_t stream) {
     case 8:
       hipLaunchKernelGGL((rmsnorm_kernel<8, ALIGNED>), grid, block, 0, stream, a);
       break;
-    case 16:
-      hipLaunchKernelGGL((rmsnorm_kernel<16, ALIGNED>), grid, block, 0, stream, a);
+    case kNormChunks:
+      hipLaunchKernelGGL((rmsnorm_kernel<kNormChunks, true>), grid, block, 0, stream, a);
       break;
     default:
       hipLaunchKernelGGL((rmsnorm_kernel<0, false>), grid, block, 0, stream, a);
