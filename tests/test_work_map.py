@@ -117,8 +117,15 @@ def test_shared_cus_with_fewer_than_8_groups(dump_bin, groups, m_blocks, group, 
 @pytest.mark.parametrize("per_cu", [2, 3])
 @pytest.mark.parametrize("groups,m_blocks,group", [(8, 11, 3), (8, 24, 4), (4, 16, 7), (64, 15, 4), (3, 40, 1)])
 def test_without_the_causal_limit(dump_bin, groups, m_blocks, group, per_cu):
-    """Items of equal length: the rotated order, whatever number of workgroups a CU holds."""
+    """Items of equal length: the rotated order, whatever number of workgroups a CU holds, and
+    launches of fewer than 8 groups take them one after the other (within a turn of the rotation)."""
     rows = _run(dump_bin, groups, m_blocks, group, 4, per_cu, 0)
-    assert rows == _run(dump_bin, groups, m_blocks, group, 4, 1, 1)  # one workgroup per CU: nothing shared
+    ilv = 4 if groups >= 8 else 1
+    assert rows == _run(dump_bin, groups, m_blocks, group, ilv, 1, 1)  # one workgroup per CU: nothing shared
+    if groups < 8:
+        order = [g for g, _ in (tuple(map(int, ln.split()[1:])) for ln in rows.splitlines()) if g >= 0]
+        assert all(abs(g - w // (m_blocks * group)) <= (w % (m_blocks * group) < 32 or
+                                                        w % (m_blocks * group) >= m_blocks * group - 32)
+                   for w, g in enumerate(order))
     done = [tuple(map(int, ln.split()[1:])) for ln in rows.splitlines()]
     assert sorted(p for p in done if p[0] >= 0) == [(g, i) for g in range(groups) for i in range(m_blocks * group)]

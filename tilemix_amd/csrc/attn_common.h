@@ -44,7 +44,13 @@ __host__ __device__ __forceinline__ int fast_div(int n, const FastDiv& f) {
 //   * for the last G % 8 groups: their items dealt over all 8 XCDs (position
 //     8 j' + x), which also covers a launch with fewer than 8 groups.  Those
 //     groups run ilv at a time as well, so that such a launch, too, starts with
-//     the long query blocks of several groups and ends on the short ones.
+//     the long query blocks of several groups and ends on the short ones.  Without
+//     the causal limit a group's items are equally long, and launches of fewer than 8
+//     groups take one at a time: each sequence's items are then spread evenly over
+//     the CUs, where several at a time (of different lengths) gave some CUs two or
+//     three of the long ones.  Kernel in us, several / one at a time: 4/1 heads x 64, 4
+//     of 475 .. 4214 tokens 130 / 75, 4 of 1386 .. 4202 133 / 97; 14/2 heads x 64, 2 of 583
+//     and 1543 (int8 mode) 42 / 31; of 80 launches none is slower beyond the repeats.
 // per_xcd (the grid is 8 * per_xcd) = (G / 8) * ipg + ceil((G % 8) * ipg / 8).
 __host__ __device__ inline int64_t work_items_per_xcd(int64_t groups, int64_t ipg) {
   return (groups / 8) * ipg + ((groups % 8) * ipg + 7) / 8;
@@ -65,8 +71,9 @@ inline WorkMap make_work_map(int total_items, int ipg, int ilv, int group, int h
                              int wgs_per_cu = 2) {
   WorkMap w;
   w.ipg = ipg;
-  w.ilv = ilv;
   w.gpx = total_items / ipg / 8;
+  if (!causal && w.gpx == 0) ilv = 1;
+  w.ilv = ilv;
   w.tail = total_items / ipg % 8;
   w.full_j = w.gpx * ipg;
   w.per_xcd = (int)work_items_per_xcd(total_items / ipg, ipg);
